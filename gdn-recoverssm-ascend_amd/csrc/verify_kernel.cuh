@@ -8,63 +8,64 @@
 //     S_t q~_t    = G_t     S_0 q~_t + sum_{s<=t} (G_t/G_s)   (k_s.q~_t) c_s
 // The state enters only through the 2Q matrix-vector products
 // S_0 [k_0 .. k_{Q-1}, q~_0 .. q~_{Q-1}], computed on the matrix cores
-// (v_mfma_f32_16x16x4_f32, FP32 in and out) from one read of the state; the
+// (v_mfma_f32_4x4x1_16b_f32, FP32 in and out) from one read of the state; the
 // per-row recurrence then runs on Q-vectors with the Gram matrix
 // k_s.{k_t, q~_t}, evaluated incrementally (no divisions):
 //     u_j <- d_t u_j + c_t (k_t.k_j),  w_j <- d_t w_j + c_t (k_t.q~_j).
 //
-// Work decomposition: one wave per (row, value head, 128-row tile of V). The
-// tile is eight 16-row MFMA blocks streamed through two register buffers: the
-// loads of blocks i+2 and i+3 are in flight while blocks i and i+1 are on the
-// matrix cores, and each 64-row half runs its recurrence while the next
-// half's loads are outstanding. Everything the recurrence needs from memory
-// (v, gates) is loaded before the first state block, because the vector memory
-// counter retires in issue order. The deferred-commit variant (DEFER) works
-// on 64-row tiles: four blocks, one recurrence.
+// Work decomposition: one wave per (row, value head, TILE rows of V), TILE =
+// 16, 64 or 128 (deferred commit: 16, 32 or 64) by the size of the launch
+// (verify_tile in verify.hip). A
+// tile is 16-row blocks streamed through two register buffers: the loads of
+// blocks i+2 and i+3 are in flight while blocks i and i+1 are on the matrix
+// cores, and each 64-row half runs its recurrence while the next half's loads
+// are outstanding. Everything the recurrence needs from memory (v, gates) is
+// loaded before the first state block, because the vector memory counter
+// retires in issue order.
 //
-// MFMA operand layout (16x16x4, wave64): A lane l = (row l%16, k-slot l/16),
-// B lane l = (k-slot l/16, column l%16), D lane l register r = (row
-// 4*(l/16)+r, column l%16). Lane (i, s) holds the 16-byte chunks 4j+s of its
-// row, so the k-slot s of MFMA (j, e) holds element E*(4j+s)+e; B uses the
-// same permutation of K. Rows read with ordinary loads are loaded in that
-// layout; rows read non-temporally (the early rows of a large batch, see
-// verify_kernel) are loaded in row runs and reach it through LDS.
+// Matrix-core layout. A 4x4x1 instruction is 16 independent blocks of a
+// 4-row by 4-column outer product: lane l = 4*kb + i holds row i of A and
+// column i of B of block kb, and register r of D holds (row r, column i).
+// Here block kb takes the 16-byte chunks 16j + kb of four state rows (A) and of
+// four of the vectors k, q~ (B), so
+//   * a load gives the 64 lanes four whole runs of 256 bytes, one per state
+//     row, straight in the operand layout (the 16x16x4 instruction's layout is
+//     16 rows x 64 bytes per load: half of 16 lines, which is why that form
+//     needed a detour through LDS for its non-temporal loads);
+//   * the B operands are the same registers for every block of rows (they
+//     were re-read from LDS for each), loaded by each lane from q and k: no
+//     LDS staging and no barrier before the first product;
+//   * 4 columns are computed, not 16, of which Q = 4 uses 8: half the
+//     matrix-core time at Q <= 4, the same at Q = 8;
+//   * the Gram matrix is the same instruction on the B registers themselves.
+// The 16 blocks' partial sums are added across lanes at the end of four rows
+// (reduce_rows: 3 lane swaps, 3 adds and 2 rotated adds per 4x4 tile).
 //
 // Template parameters: S state element type, A activation type (q, k, v and
 // the key record / output when they share it), J 16-byte chunks per lane per
-// row (K <= 4*E*J), QM window capacity (Q <= QM).
+// row (K <= 16*E*J), QM window capacity (Q <= QM).
 #pragma once
 
 #include "gdn_common.cuh"
 
 namespace gdn {
 
+// Element strides and page counts fit in 32 bits (checked on the host); every
+// product with a row, token or page index is formed in 64 bits. The arguments
+// that a wave needs before its first state load come first (see `hold` in
+// verify_wave), those of the deferred commit next.
 struct VerifyArgs {
+  const void *qsl, *indices;
   const void *q, *k, *v, *g, *beta;
   const void *state;
-  float *corr;
-  void *key;
-  float *decay;
-  void *out;
-  const void *qsl, *indices;
-  // Element strides and page counts fit in 32 bits (checked on the host);
-  // every product with a row, token or page index is formed in 64 bits.
+  int32_t qsl_s, idx_s, qsl_i64, idx_i64;  // index dtypes: 1 for int64
+  int32_t NVT, ratio;                      // tiles of a (row, value head); value heads per head
+  uint32_t nvt_magic, ratio_magic;         // udiv_magic of each
   int32_t state_bs, q_ts, k_ts, v_ts, g_ts, beta_ts;
-  int32_t corr_rs, key_rs, decay_rs, out_ts;
-  int32_t qsl_s, idx_s;
-  int32_t blocks, null_block;
-  int32_t tokens, heads, value_heads, Q, record_rows;
   int32_t state_hs, state_vs;
-  int32_t corr_hs, corr_ts, key_hs, key_ts, decay_hs, decay_ts;
-  float scale;
-  int32_t K, V, NVT;
-  int32_t qsl_i64, idx_i64;                  // index dtypes: 1 for int64
-  int32_t g_f32, beta_f32, key_f32, out_f32;  // 1: FP32, 0: activation dtype
-  int32_t l2norm, key_per_value_head;
-  // Fused gating: g and beta hold the raw projections a and b.
-  const void *a_log, *dt_bias;
-  int32_t gated, a_log_dt, dt_bias_dt;
-  float softplus_beta, softplus_threshold;
+  int32_t blocks, null_block, tokens, Q, K, V;
+  int32_t g_f32, beta_f32;  // 1: FP32, 0: activation dtype
+  int32_t nt_rows;          // rows b < nt_rows read their state non-temporally
   // Deferred commit (kernels instantiated with DEFER): for every current row
   // the pending row it continues (p_rows), the previous step's plan arrays
   // indexed by pending row, and that step's records.
@@ -74,31 +75,36 @@ struct VerifyArgs {
   int32_t p_corr_rs, p_key_rs, p_decay_rs;
   int32_t p_corr_hs, p_corr_ts, p_key_hs, p_key_ts, p_decay_hs, p_decay_ts;
   int32_t p_key_f32, p_key_per_value_head, p_record_rows, p_num_rows;
-  int32_t nt_rows;  // rows b < nt_rows read their state non-temporally
+  // Read after the state loads are issued.
+  float *corr;
+  void *key;
+  float *decay;
+  void *out;
+  int32_t corr_rs, key_rs, decay_rs, out_ts;
+  int32_t record_rows;
+  int32_t corr_hs, corr_ts, key_hs, key_ts, decay_hs, decay_ts;
+  float scale;
+  int32_t key_f32, out_f32;
+  int32_t l2norm, key_per_value_head;
+  // Fused gating: g and beta hold the raw projections a and b.
+  const void *a_log, *dt_bias;
+  int32_t gated, a_log_dt, dt_bias_dt;
+  float softplus_beta, softplus_threshold;
 };
 
+// Division of x < 2^32 by a runtime d >= 1 with m = floor((2^32 - 1) / d): the
+// high product is x / d rounded down or one less, so one correction makes it
+// exact. Five scalar instructions for a uniform x; the compiler's division
+// is a chain of about twenty through the vector reciprocal.
+inline uint32_t udiv_magic(uint32_t d) { return 0xffffffffu / d; }
+__host__ __device__ inline uint32_t udiv(uint32_t x, uint32_t d, uint32_t m) {
+  const uint32_t q = uint32_t((uint64_t(x) * m) >> 32);
+  return x - q * d >= d ? q + 1 : q;
+}
+
 constexpr int kVerifyThreads = 64;  // one wave per (row, value head, tile)
-constexpr int kTileRows = 128;     // eight MFMA row blocks of 16 rows
-// The deferred-commit kernels stream half tiles: a wave that also stores the
-// folded state lives twice as long per row, and with twice as many, shorter
-// waves the launch's tail is shorter (measured: 232 against 236 us per step;
-// the plain verify is 3 us faster with whole tiles).
-constexpr int kDeferTileRows = 64;
-// One 16-row block of the state tile on its way from the row-contiguous load
-// layout to the matrix-core operand layout: 16 rows x 4J chunks of 16 bytes.
-// It is staged in two rounds of half the row's chunks (one for J = 1), so the
-// stage holds 16 rows x 2J chunks.
-__host__ __device__ constexpr int verify_stage_rounds(int j) { return j >= 2 ? 2 : 1; }
-__host__ __device__ constexpr int verify_stage_bytes(int j) { return 16 * (4 * j / verify_stage_rounds(j)) * 16; }
-extern __shared__ __align__(16) uint32_t verify_stage[][4];
-__host__ __device__ constexpr int verify_tile_rows(bool deferred) { return deferred ? kDeferTileRows : kTileRows; }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename A>
-__device__ __forceinline__ float ld_act(const void *p, int64_t i) {
-  return to_f32(static_cast<const A *>(p)[i]);
-}
 
 template <typename A>
 __device__ __forceinline__ void st_f32_or(void *p, int64_t i, bool f32, float x) {
@@ -130,28 +136,73 @@ __device__ __forceinline__ float bits_to_f32(uint32_t u) {
     return to_f32(__builtin_bit_cast(A, uint16_t(u)));
 }
 
-// One activation element at a byte offset (kOutOfRange reads 0); imm is a
-// constant byte displacement applied only to in-range offsets.
+// One activation element at a byte offset (kOutOfRange reads 0).
 template <typename A>
-__device__ __forceinline__ float buf_ld_act(__amdgpu_buffer_rsrc_t r, int byte_off, int imm = 0) {
+__device__ __forceinline__ float buf_ld_act(__amdgpu_buffer_rsrc_t r, int byte_off) {
   if constexpr (sizeof(A) == 4)
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 0));
   else
-    return bits_to_f32<A>(__builtin_amdgcn_raw_buffer_load_b16(r, byte_off + imm, 0, 0));
+    return bits_to_f32<A>(__builtin_amdgcn_raw_buffer_load_b16(r, byte_off, 0, 0));
 }
 
-// Four consecutive activation elements starting at a byte offset: one 16-byte
-// load for FP32 (dword alignment suffices), four 2-byte loads otherwise, which
-// need no alignment beyond the element's.
-template <typename A>
-__device__ __forceinline__ void buf_ld4_act(__amdgpu_buffer_rsrc_t r, int byte_off, float *x) {
+// N (4 or 8) consecutive elements of a tensor that is only aligned to its
+// elements. `WordRsrc` starts at the dword holding the first byte; 16-bit
+// elements are read as the N/2 dwords from the one holding the first element
+// and, where the run starts in a dword's upper half, one more; a funnel shift
+// lines them up. Every dword read holds an element of the run.
+struct WordRsrc {
+  __amdgpu_buffer_rsrc_t r;
+  int skip;  // bytes from the resource's start to the tensor's first byte (0 or 2)
+};
+__device__ __forceinline__ WordRsrc make_word_rsrc(const void *p, int64_t byte_off) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p) + uintptr_t(byte_off);
+  return {make_rsrc(reinterpret_cast<const void *>(at & ~uintptr_t(3)), 0), int(at & 2)};
+}
+template <typename A, int N>
+struct RawRun {
+  uint32_t w[sizeof(A) == 4 ? N : N / 2 + 1];
+  int sh;
+};
+template <typename A, int N>
+__device__ __forceinline__ void load_run(const WordRsrc &b, int byte_off, bool live, RawRun<A, N> &x) {
+  const int off = byte_off + b.skip;
   if constexpr (sizeof(A) == 4) {
-    const auto u = __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, 0);
-    x[0] = __uint_as_float(u[0]), x[1] = __uint_as_float(u[1]);
-    x[2] = __uint_as_float(u[2]), x[3] = __uint_as_float(u[3]);
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+      const auto u = __builtin_amdgcn_raw_buffer_load_b128(b.r, live ? off + i * 4 : kOutOfRange, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x.w[i + e] = u[e];
+    }
+  } else {
+    const int at = live ? off & ~3 : kOutOfRange;
+    const bool odd = (off & 2) != 0;
+    if constexpr (N == 4) {
+      const auto u = __builtin_amdgcn_raw_buffer_load_b64(b.r, at, 0, 0);
+      x.w[0] = u[0], x.w[1] = u[1];
+    } else {
+      const auto u = __builtin_amdgcn_raw_buffer_load_b128(b.r, at, 0, 0);
+      x.w[0] = u[0], x.w[1] = u[1], x.w[2] = u[2], x.w[3] = u[3];
+    }
+    x.w[N / 2] = 0u;
+    // A branch of the wave: rare, and skipping it leaves fewer loads between
+    // the others and the wait for them, never more.
+    if (__builtin_amdgcn_ballot_w64(odd) != 0)
+      x.w[N / 2] = __builtin_amdgcn_raw_buffer_load_b32(b.r, live && odd ? at + N * 2 : kOutOfRange, 0, 0);
+    x.sh = odd ? 16 : 0;
+  }
+}
+template <typename A, int N>
+__device__ __forceinline__ void unpack_run(const RawRun<A, N> &x, float (&out)[N]) {
+  if constexpr (sizeof(A) == 4) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] = __uint_as_float(x.w[e]);
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = buf_ld_act<A>(r, byte_off, i * 2);
+    for (int i = 0; i < N / 2; ++i) {
+      const uint32_t u = __builtin_amdgcn_alignbit(x.w[i + 1], x.w[i], x.sh);
+      out[2 * i] = bits_to_f32<A>(u & 0xffffu);
+      out[2 * i + 1] = bits_to_f32<A>(u >> 16);
+    }
   }
 }
 
@@ -198,6 +249,33 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The sum over the 16 blocks kb = lane / 4 of a value per (block, lane % 4),
+// in every lane.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+constexpr int kRowRor8 = 0x128, kRowRor4 = 0x124;  // rotations inside 16 lanes
+__device__ __forceinline__ float swap_add32(float x, float y) {  // lanes 0-31: x summed over the halves; 32-63: y
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float swap_add16(float x, float y) {  // even 16-lane rows: x summed over row pairs; odd: y
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float sum_blocks(float x) {
+  x = swap_add32(x, x);
+  x = swap_add16(x, x);
+  return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
+}
+// The same for the four registers of a 4x4 result tile at once: lane
+// 16*r + 4*any + i gets the sum of row r, column i.
+__device__ __forceinline__ float reduce_rows(f32x4 a) {
+  const float x = swap_add16(swap_add32(a[0], a[2]), swap_add32(a[1], a[3]));
+  return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
+}
+
 // DEFER: before verifying, apply the previous step's commit for this row (the
 // fold of kernels.py:1222-1324, folded into the next verify): the state comes
 // from the pending commit's source page, its accepted prefix is replayed from
@@ -207,36 +285,42 @@ __device__ __forceinline__ void wave_lds_sync() {
 // the stored page is. Each state page is read once per step instead of twice.
 // The wave's LDS, declared once per kernel and shared by both cache-policy
 // bodies below (a __shared__ array inside each would be allocated twice).
-// The non-temporal body also stages state blocks in dynamic LDS
-// (verify_stage_bytes), given to the launch only when it has such rows.
-template <int QM, int KP, int J, bool DEFER>
-struct VerifyLds {
-  float m[2 * QM][KP + 4];  // k and q~ vectors, row pitch KP + 4 (bank spread)
-  float gram[QM][2 * QM];
-  float d[64][2 * QM + 1];  // GEMV results of one 64-row half tile
-  float inv[2 * QM];
+template <int QM, int KP, bool DEFER, int TILE>
+struct __align__(16) VerifyLds {
+  static constexpr int HALF = TILE < 64 ? TILE : 64;
+  float d[HALF][2 * QM + 1];  // GEMV results of one half tile
   __align__(16) float pk[DEFER ? QM : 1][DEFER ? KP : 1];  // pending commit's keys
+  float pc[DEFER ? QM : 1][DEFER ? HALF : 1];              // and its corrections of the tile's rows
 };
 
-template <typename S, typename A, int J, int QM, bool DEFER, bool NT>
-__device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4 * Chunk<S>::E * J, J, DEFER> &L) {
+template <typename S, typename A, int J, int QM, bool DEFER, bool NT, int TILE>
+__device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 16 * Chunk<S>::E * J, DEFER, TILE> &L) {
+  static_assert(!DEFER || TILE <= 64, "the pending corrections cover one half tile");
   constexpr int E = Chunk<S>::E;       // elements per 16-byte chunk
-  constexpr int KP = 4 * E * J;        // K padded to 4 k-slots x J chunks x E
-  constexpr int NV = 2 * QM;           // used MFMA columns (<= 16)
-  constexpr int TILE = verify_tile_rows(DEFER);
-  constexpr int NRB = TILE / 16;  // 16-row MFMA blocks per tile (8 or 4)
-  auto &m_lds = L.m;
-  auto &gram_lds = L.gram;
+  constexpr int KP = 16 * E * J;       // K padded to 16 blocks x J chunks x E
+  constexpr int NV = 2 * QM;           // columns: k_0 .. k_{QM-1}, q~_0 .. q~_{QM-1}
+  constexpr int CG = (NV + 3) / 4;     // groups of 4 columns
+  constexpr int CGK = (QM + 3) / 4;    // column groups that hold a k
+  constexpr int NRB = TILE / 16;       // 16-row blocks per tile
+  constexpr int HALF = TILE < 64 ? TILE : 64;  // rows of one recurrence (one per lane)
+  constexpr int HRB = HALF / 16;
   auto &d_lds = L.d;
-  auto &inv_lds = L.inv;
   auto &pk_lds = L.pk;
+  auto &pc_lds = L.pc;
 
-  const int nvt = a.NVT;
-  const int hv = int(blockIdx.x) / nvt;
-  const int vt = int(blockIdx.x) - hv * nvt;
+  // One batch of argument reads: left to itself the compiler reads each
+  // argument where it is first used, one wait per read, ahead of the state
+  // loads. The asm is one consumer of them all.
+  asm volatile("" ::"s"(a.qsl), "s"(a.indices), "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.g), "s"(a.beta), "s"(a.state),
+               "s"(a.qsl_s), "s"(a.idx_s), "s"(a.qsl_i64), "s"(a.idx_i64), "s"(a.NVT), "s"(a.ratio), "s"(a.nvt_magic),
+               "s"(a.ratio_magic), "s"(a.state_bs), "s"(a.q_ts), "s"(a.k_ts), "s"(a.v_ts), "s"(a.g_ts),
+               "s"(a.beta_ts), "s"(a.state_hs), "s"(a.state_vs), "s"(a.blocks), "s"(a.null_block), "s"(a.tokens),
+               "s"(a.Q), "s"(a.K), "s"(a.V));
+  const int hv = int(udiv(blockIdx.x, uint32_t(a.NVT), a.nvt_magic));
+  const int vt = int(blockIdx.x) - hv * a.NVT;
   const int b = int(blockIdx.y);
-  const int ratio = a.value_heads / a.heads;
-  const int h = hv / ratio;
+  const int ratio = a.ratio;
+  const int h = int(udiv(uint32_t(hv), uint32_t(ratio), a.ratio_magic));
   const int lane = threadIdx.x;
   const int V = a.V, K = a.K;
   const int row0 = vt * TILE;
@@ -315,7 +399,11 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
                                       int64_t(dt) * a.p_decay_ts) * 4);
       addr = dt >= 0 && dt < QM ? (dt < Q ? da : any_word) : addr;
     }
-    gw = lane_word(addr & ~uintptr_t(3));
+    // A relaxed atomic load is an ordinary one that the compiler leaves here: it
+    // moved the plain load down to its use, behind the state loads, and waiting
+    // for it was then waiting for all of them.
+    gw = __hip_atomic_load(reinterpret_cast<const __attribute__((address_space(1))) uint32_t *>(addr & ~uintptr_t(3)),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
   }
 
   // Pending commit of the previous step (same validity rule as the fold,
@@ -358,58 +446,62 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
   const bool verify_row = !null_slot && valid_mask != 0;
   if (!verify_row) valid_mask = 0;
 
-  const int li = lane & 15, ls = lane >> 4;  // MFMA row / column index and k-slot
+  const int kb = lane >> 2, ij = lane & 3;     // block; state row / column within its 4
+  const int q16 = lane >> 4, bq = kb & 3;      // after reduce_rows: state row, and the copy's number
 
-  // ---- 2. small loads first: k/q chunks, v of the lane's rows ----
-  constexpr int C4 = KP / 4;  // 4-element chunks per vector
-  constexpr int STAGE_PASSES = (NV * C4 + kVerifyThreads - 1) / kVerifyThreads;
-  // DEFER: the pending commit's keys (token t, element kk) for LDS, FP32 or
-  // activation-typed records (one of the two loads reads out of range).
+  // ---- 2. small loads first: the lane's chunks of k and q, v of its rows ----
+  // Column c = 4*cg + ij is k_c, or q_{c - QM}.
+  const WordRsrc rq = make_word_rsrc(a.q, bos * a.q_ts * AS), rk = make_word_rsrc(a.k, bos * a.k_ts * AS);
+  RawRun<A, E> raw_q[CG][J], raw_k[CG][J];
+#pragma unroll
+  for (int cg = 0; cg < CG; ++cg) {
+    const int col = 4 * cg + ij;
+    const bool is_q = col >= QM;
+    const int t = (is_q ? col - QM : col) & 31;
+    // Non-short-circuit tests: a short-circuit chain became a branch per load,
+    // with kernel arguments reloaded inside it.
+    const bool on = (col < NV) & (((valid_mask >> t) & 1u) != 0);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int kk = (16 * j + kb) * E;
+      const int off = (t * (is_q ? a.q_ts : a.k_ts) + h * K + kk) * AS;
+      // With QM a multiple of 4 a group is all k or all q; else one of two
+      // loads reads out of range.
+      if (QM % 4 != 0 || 4 * cg < QM) load_run<A, E>(rk, off, on & !is_q & (kk < K), raw_k[cg][j]);
+      if (QM % 4 != 0 || 4 * cg >= QM) load_run<A, E>(rq, off, on & is_q & (kk < K), raw_q[cg][j]);
+    }
+  }
+  // DEFER: the pending commit's keys (token t, 4 elements from kk) for LDS, FP32
+  // or activation-typed records (one of the two loads reads out of range),
+  // and its corrections of the lane's row.
+  constexpr int C4 = KP / 4;
   constexpr int PK_PASSES = DEFER ? (QM * C4 + kVerifyThreads - 1) / kVerifyThreads : 1;
-  float pkx[PK_PASSES][4];
+  RawRun<float, 4> pk32[PK_PASSES];
+  RawRun<A, 4> pka[PK_PASSES];
+  float pcx[QM];
   if constexpr (DEFER) {
     const int key_head = a.p_key_per_value_head ? hv : h;
     const int64_t kbase = int64_t(prow) * a.p_key_rs + int64_t(key_head) * a.p_key_hs;
     const bool kf32 = a.p_key_f32 != 0;
-    const __amdgpu_buffer_rsrc_t rpk = make_rsrc(a.p_key, kbase * (kf32 ? 4 : AS));
+    const WordRsrc rpk = make_word_rsrc(a.p_key, kbase * (kf32 ? 4 : AS));
     int lim = pend_len;
-    asm volatile("" : "+v"(lim));  // per-lane select, not a branch (see load_block)
+    asm volatile("" : "+v"(lim));  // per-lane select, not a branch
 #pragma unroll
     for (int p = 0; p < PK_PASSES; ++p) {
       const int idx = p * kVerifyThreads + lane;
       const int t = idx / C4, kk = (idx - t * C4) * 4;
-      const bool live = t < lim && kk < K;
+      const bool live = (t < lim) & (kk < K);
       const int el = t * a.p_key_ts + kk;
-      float x32[4], xa[4];
-      buf_ld4_act<float>(rpk, live && kf32 ? el * 4 : kOutOfRange, x32);
-      buf_ld4_act<A>(rpk, live && !kf32 ? el * AS : kOutOfRange, xa);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pkx[p][e] = x32[e] + xa[e];
+      load_run<float, 4>(rpk, el * 4, live & kf32, pk32[p]);
+      load_run<A, 4>(rpk, el * AS, live & !kf32, pka[p]);
     }
-  }
-  const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.q, bos * a.q_ts * AS), rk = make_rsrc(a.k, bos * a.k_ts * AS);
-  float xs[STAGE_PASSES][4];
+    const __amdgpu_buffer_rsrc_t rpc =
+        make_rsrc(a.p_corr, (int64_t(prow) * a.p_corr_rs + int64_t(hv) * a.p_corr_hs + row0) * 4);
+    const int row_lim = ((lane < HALF) & (row0 + lane < V)) ? lim : 0;
 #pragma unroll
-  for (int p = 0; p < STAGE_PASSES; ++p) {
-    const int idx = p * kVerifyThreads + lane;
-    const int vid = idx / C4, kk = (idx - vid * C4) * 4;
-    const bool is_q = vid >= QM;
-    const int t = (is_q ? vid - QM : vid) & 31;
-    // Non-short-circuit tests: a short-circuit chain became a branch per pass,
-    // with kernel arguments reloaded inside it.
-    const bool live = (vid < NV) & (((valid_mask >> t) & 1u) != 0) & (kk < K);
-    const int el = t * (is_q ? a.q_ts : a.k_ts) + h * K + kk;
-    const int off = live ? el * AS : kOutOfRange;
-    if constexpr (C4 * QM % kVerifyThreads == 0) {
-      // Every pass lies wholly inside the k vectors or wholly inside the q ones.
-      buf_ld4_act<A>(p * kVerifyThreads < C4 * QM ? rk : rq, off, xs[p]);
-    } else {
-      float xq[4], xk[4];
-      buf_ld4_act<A>(rq, is_q ? off : kOutOfRange, xq);
-      buf_ld4_act<A>(rk, is_q ? kOutOfRange : off, xk);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) xs[p][e] = xq[e] + xk[e];
-    }
+    for (int t = 0; t < QM; ++t)
+      pcx[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+          rpc, t < row_lim ? (t * a.p_corr_ts + lane) * 4 : kOutOfRange, 0, 0));
   }
   // v of the lane's row in each half; the second half is loaded later, after
   // the loads it must not wait behind.
@@ -419,7 +511,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
 #pragma unroll
     for (int t = 0; t < QM; ++t) {
       const int vr = row0 + half * 64 + lane;
-      const bool ok = (vr < V) & (((valid_mask >> t) & 1u) != 0);
+      const bool ok = (vr < V) & (lane < HALF) & (((valid_mask >> t) & 1u) != 0);
       const int off = ok ? (t * int(a.v_ts) + int(out_base) + half * 64 + lane) * AS : kOutOfRange;
       vv[half][t] = buf_ld_act<A>(rv, off);
     }
@@ -427,22 +519,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
   load_v(0);
 
   // ---- 3. first two state blocks ----
-  // Buffer loads: one resource per (slot, head) tile and a 32-bit per-lane
-  // offset per chunk. Rows >= V lie past the resource's extent and read as
-  // zero; chunks >= K get an out-of-range offset.
-  // Ordinary loads (NT false) read the operand layout directly: load j of
-  // block rb gives lane (li, ls) chunk 4j + ls of row rb*16 + li, 16 rows x
-  // 64 bytes per load. Non-temporal loads that touch half of each of 16 lines
-  // fetched lines twice and ran slower than ordinary ones (131 against 116 us
-  // for the B=256 tiles alone), so the non-temporal body (NT) reads rows in
-  // long runs: a block is 16 rows x CPR 16-byte chunks (CPR = 4J, the padded
-  // row), staged through LDS into the operand layout in ROUNDS rounds of SC =
-  // CPR / ROUNDS chunks per row (`transpose` below; with ordinary loads that
-  // detour cost 4 us). Load j belongs to round g = j / JR and gives lane l the
-  // chunk (row (j % JR)*RPL + l/SC, chunk g*SC + l%SC): 4 rows x 256 bytes per
-  // load at K = 128 FP32 (whole rows measured 102 us for the same tiles, runs
-  // of 256 bytes 104 us, and halving the stage keeps the LDS from limiting
-  // the waves per CU).
+  // Buffer loads: one resource per (slot, head) tile, a 32-bit per-lane offset
+  // per chunk and the block step in the scalar offset. Rows >= V lie past the
+  // resource's extent and read as zero; chunks >= K get an out-of-range offset.
+  // Register g*J + j of a block: row 4g + ij, chunk 16j + kb.
   const int tile_rows = V - row0 < TILE ? V - row0 : TILE;
   const int tile_bytes = tile_rows * a.state_vs * int(sizeof(S));
   auto tile_rsrc = [&](int64_t page, bool use) {
@@ -460,105 +540,48 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
   // A 24-bit product (row_bytes < 2^24, checked on the host): a full multiply
   // here became a 64-bit multiply-add whose unused high addend was a register
   // with a load in flight, and waiting for it held back the first state loads.
-  const int lane_off = int(__umul24(unsigned(li), unsigned(row_bytes))) + ls * 16;
-  constexpr int CPR = 4 * J;                 // 16-byte chunks per padded row (J <= 16)
-  constexpr int ROUNDS = verify_stage_rounds(J);
-  constexpr int SC = CPR / ROUNDS;           // chunks of each row staged per round
-  constexpr int JR = J / ROUNDS;             // loads (and operand registers) per round
-  constexpr int RPL = 64 / SC;               // rows per load
-  const int c_chunk = lane & (SC - 1), c_row = lane / SC;
-  const int c_off = int(__umul24(unsigned(c_row), unsigned(row_bytes))) + c_chunk * 16;
-  const int load_step = RPL * row_bytes;
-  // Lane offset of load j (its round's chunks past K read and write nothing)
-  // and the uniform part that rides in soffset.
-  auto c_voff = [&](int j) { return ((j / JR) * SC + c_chunk) * E < K ? c_off : kOutOfRange; };
-  auto c_soff = [&](int rb, int j) { return rb * 16 * row_bytes + (j % JR) * load_step + (j / JR) * SC * 16; };
-  // The pending corrections of the lane's row, fetched with each block.
-  const __amdgpu_buffer_rsrc_t rpc =
-      make_rsrc(a.p_corr, (int64_t(prow) * a.p_corr_rs + int64_t(hv) * a.p_corr_hs + row0) * 4);
+  const int lane_off = int(__umul24(unsigned(ij), unsigned(row_bytes))) + kb * 16;
+  constexpr int BR = 4 * J;  // registers (16-byte chunks per lane) of a block
+  auto s_voff = [&](int j) { return (16 * j + kb) * E < K ? lane_off : kOutOfRange; };
+  auto s_soff = [&](int rb, int g, int j) { return (rb * 16 + 4 * g) * row_bytes + j * 256; };
   // One form for every K, and every block is loaded (blocks past V read as
   // zero): a conditional load would leave a path on which it was not issued,
   // and the wait counts of every later MFMA would have to assume that path,
   // draining the pipeline at each block.
-  auto load_block = [&](int rb, uint4 (&dst)[J], float (&pc)[QM]) {
-    // The block step rides in soffset, which the range check covers as well.
+  auto load_block = [&](int rb, uint4 (&dst)[BR]) {
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      if constexpr (NT) {
-        dst[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, c_voff(j), c_soff(rb, j), kPolicyNT));
-      } else {
-        const int vo = (4 * j + ls) * E < K ? lane_off + j * 64 : kOutOfRange;
-        dst[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, vo, rb * 16 * row_bytes, 0));
-      }
-    }
-    if constexpr (DEFER) {
-      const int v = rb * 16 + li;
-      // Tokens to replay as a per-lane value: a select on it stays a select
-      // (a wave-uniform bound would turn each load into a branch).
-      int lim = row0 + v < V ? pend_len : 0;
-      asm volatile("" : "+v"(lim));
+    for (int g = 0; g < 4; ++g)
 #pragma unroll
-      for (int t = 0; t < QM; ++t)
-        pc[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-            rpc, t < lim ? (t * a.p_corr_ts + v) * 4 : kOutOfRange, 0, 0));
-    }
+      for (int j = 0; j < J; ++j)
+        dst[g * J + j] = __builtin_bit_cast(
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, s_voff(j), s_soff(rb, g, j), NT ? kPolicyNT : 0));
   };
-  // Row-run block -> operand layout through LDS, one round at a time. In a
-  // round, chunk c (of the round's SC) of block row r sits at r*SC +
-  // (c ^ swz(r)): the 64 lanes of a write cover 64 consecutive slots, and the
-  // 16 lanes (li = 0..15) of a read that share ls hit 16 distinct 16-byte
-  // bank groups. Operand register j (chunk 4j + ls) belongs to round j / JR.
-  constexpr int SWZ_MASK = (SC < 16 ? SC : 16) - 1;
-  constexpr int SWZ_SH = SC >= 16 ? 0 : SC == 8 ? 1 : 2;
-  auto swz = [](int r) { return (r >> SWZ_SH) & SWZ_MASK; };
-  auto row_slot = [&](int j) {  // slot of load j's chunk
-    const int r = (j % JR) * RPL + c_row;
-    return r * SC + (c_chunk ^ swz(r));
-  };
-  auto op_slot = [&](int j) { return li * SC + ((4 * (j % JR) + ls) ^ swz(li)); };  // slot of operand register j
-  auto stage_write = [&](const uint4 (&buf)[J], int g) {
-#pragma unroll
-    for (int j = g * JR; j < (g + 1) * JR; ++j) *reinterpret_cast<uint4 *>(verify_stage[row_slot(j)]) = buf[j];
-  };
-  auto stage_read = [&](uint4 (&buf)[J], int g) {
-#pragma unroll
-    for (int j = g * JR; j < (g + 1) * JR; ++j) buf[j] = *reinterpret_cast<const uint4 *>(verify_stage[op_slot(j)]);
-  };
-  auto transpose = [&](uint4 (&buf)[J]) {
-    if constexpr (NT) {
-#pragma unroll
-      for (int g = 0; g < ROUNDS; ++g) {
-        stage_write(buf, g);
-        wave_lds_sync();
-        stage_read(buf, g);
-        wave_lds_sync();  // the next round's writes stay behind these reads
-      }
-    }
-  };
-  uint4 bufA[J], bufB[J];
-  float pcA[QM], pcB[QM];
-  load_block(0, bufA, pcA);
+  uint4 bufA[BR], bufB[BR];
+  __builtin_amdgcn_sched_barrier(0);  // the gates' load (and every other small one) stays ahead of the state
+  load_block(0, bufA);
   __builtin_amdgcn_sched_barrier(0);  // keep block 0's loads ahead of block 1's
-  load_block(1, bufB, pcB);
+  if constexpr (NRB > 1) load_block(1, bufB);
+  // The rest, with the arguments it needs behind `z`.
+  auto rest = [&](const auto *z) __attribute__((always_inline)) {
   float dec[QM], bet[QM];
   float neg_a = 0.0f, dtb = 0.0f;
-  if (a.gated) {
-    neg_a = -expf(scalar_param<A>(a.a_log, hv, a.a_log_dt));
-    dtb = scalar_param<A>(a.dt_bias, hv, a.dt_bias_dt);
+  if (z->gated) {
+    neg_a = -expf(scalar_param<A>(z->a_log, hv, z->a_log_dt));
+    dtb = scalar_param<A>(z->dt_bias, hv, z->dt_bias_dt);
   }
   {
     // Each gate lane decodes its own word; the window's decays and betas then
     // reach every lane by readlane.
-    const bool f32 = gate_lane_b ? a.beta_f32 != 0 : a.g_f32 != 0;
+    const bool f32 = gate_lane_b ? z->beta_f32 != 0 : z->g_f32 != 0;
     float x = f32 ? __uint_as_float(gw) : bits_to_f32<A>((gw >> gate_sh) & 0xffffu);
-    if (a.gated) {
+    if (z->gated) {
       // docs/reference/recoverssm_gdn_upstream.py:135-151
       if (gate_lane_b) {
         x = 1.0f / (1.0f + expf(-x));
       } else {
         const float xb = x + dtb;
-        const float bx = a.softplus_beta * xb;
-        const float sp = bx <= a.softplus_threshold ? log1pf(expf(bx)) / a.softplus_beta : xb;
+        const float bx = z->softplus_beta * xb;
+        const float sp = bx <= z->softplus_threshold ? log1pf(expf(bx)) / z->softplus_beta : xb;
         x = neg_a * sp;
       }
     }
@@ -571,123 +594,174 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
     }
   }
 
-  // ---- 4. stage vectors and records ----
-  const bool rec_ok = b < a.record_rows;
-  const bool key_writer = rec_ok && vt == 0 && (a.key_per_value_head || (hv % ratio) == 0);
-  const int key_head = a.key_per_value_head ? hv : h;
-  const bool key_f32 = a.key_f32 != 0;
+  // ---- 4. operands, records, Gram matrix ----
+  const bool rec_ok = b < z->record_rows;
+  const bool key_writer = rec_ok && vt == 0 && (z->key_per_value_head || hv == h * ratio);
+  float m[CG][J][E];  // the lane's chunks of its columns' vectors (B operands)
 #pragma unroll
-  for (int p = 0; p < STAGE_PASSES; ++p) {
-    const int idx = p * kVerifyThreads + lane;
-    const int vid = idx / C4, kk = (idx - vid * C4) * 4;
-    if (vid < NV) {
-      const bool is_q = vid >= QM;
-      const float sc = (is_q && !a.l2norm) ? a.scale : 1.0f;
+  for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) m_lds[vid][kk + e] = xs[p][e] * sc;
-      const int t = is_q ? vid - QM : vid;
-      if (!is_q && !a.l2norm && key_writer && ((valid_mask >> t) & 1u) && kk < K) {
-        const int64_t base = int64_t(b) * a.key_rs + int64_t(key_head) * a.key_hs + int64_t(t) * a.key_ts + kk;
+    for (int j = 0; j < J; ++j) {
+      if constexpr (QM % 4 != 0) {
+        float xk[E], xq[E];
+        unpack_run<A, E>(raw_k[cg][j], xk);
+        unpack_run<A, E>(raw_q[cg][j], xq);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) st_f32_or<A>(a.key, base + e, key_f32, xs[p][e]);
+        for (int e = 0; e < E; ++e) m[cg][j][e] = xk[e] + xq[e];
+      } else {
+        unpack_run<A, E>(4 * cg < QM ? raw_k[cg][j] : raw_q[cg][j], m[cg][j]);
       }
     }
+  if (z->l2norm) {
+    // kernels.py:645-648: x * rsqrt(sum(x*x) + 1e-6) for q and k, then q *= scale.
+#pragma unroll
+    for (int cg = 0; cg < CG; ++cg) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int e = 0; e < E; ++e) ss = __builtin_fmaf(m[cg][j][e], m[cg][j][e], ss);
+      const float inv = rsqrtf(sum_blocks(ss) + 1e-6f);
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int e = 0; e < E; ++e) m[cg][j][e] *= inv;
+    }
+  }
+  if (key_writer) {
+    const int key_head = z->key_per_value_head ? hv : h;
+    const bool key_f32 = z->key_f32 != 0;
+#pragma unroll
+    for (int cg = 0; cg < CGK; ++cg) {
+      const int t = 4 * cg + ij;
+      if (t < QM && ((valid_mask >> (t & 31)) & 1u)) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int kk = (16 * j + kb) * E;
+          if (kk < K) {
+            const int64_t base = int64_t(b) * z->key_rs + int64_t(key_head) * z->key_hs + int64_t(t) * z->key_ts + kk;
+#pragma unroll
+            for (int e = 0; e < E; ++e) st_f32_or<A>(z->key, base + e, key_f32, m[cg][j][e]);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int cg = QM / 4; cg < CG; ++cg) {
+    const float sc = 4 * cg + ij >= QM ? z->scale : 1.0f;
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int e = 0; e < E; ++e) m[cg][j][e] *= sc;
   }
   if (rec_ok && vt == 0) {
     float dl = 1.0f;
 #pragma unroll
     for (int t = 0; t < QM; ++t) dl = lane == t ? dec[t] : dl;
     if (lane < QM && ((valid_mask >> lane) & 1u))
-      a.decay[int64_t(b) * a.decay_rs + int64_t(hv) * a.decay_hs + int64_t(lane) * a.decay_ts] = dl;
+      z->decay[int64_t(b) * z->decay_rs + int64_t(hv) * z->decay_hs + int64_t(lane) * z->decay_ts] = dl;
   }
-  // DEFER: the pending keys to LDS, the pending decays to scalars.
+  // k_s . column c of lane 16*(s % 4) + c % 4 of gram[s / 4][c / 4].
+  float gram[CGK][CG];
+#pragma unroll
+  for (int s = 0; s < CGK; ++s)
+#pragma unroll
+    for (int cg = 0; cg < CG; ++cg) {
+      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(m[s][j][e], m[cg][j][e], acc, 0, 0, 0);
+      gram[s][cg] = reduce_rows(acc);
+    }
+  auto dot = [&](int s, int c) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gram[s / 4][c / 4]), 16 * (s & 3) + (c & 3)));
+  };
+  // DEFER: the pending keys and corrections to LDS, the decays to scalars. A
+  // lane's chunks of the keys stay in registers where they are few.
+  constexpr bool PK_REGS = DEFER && QM * J * E <= 32;
   float pdec[QM];
+  float pkr[PK_REGS ? QM : 1][PK_REGS ? J : 1][E];
   if constexpr (DEFER) {
 #pragma unroll
     for (int p = 0; p < PK_PASSES; ++p) {
       const int idx = p * kVerifyThreads + lane;
       const int t = idx / C4, kk = (idx - t * C4) * 4;
+      float x32[4], xa[4];
+      unpack_run<float, 4>(pk32[p], x32);
+      unpack_run<A, 4>(pka[p], xa);
       if (t < QM) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pk_lds[t][kk + e] = pkx[p][e];
+        for (int e = 0; e < 4; ++e) pk_lds[t][kk + e] = x32[e] + xa[e];
       }
     }
 #pragma unroll
     for (int t = 0; t < QM; ++t) {
+      if (lane < HALF) pc_lds[t][lane] = pcx[t];
       const bool live = pend && t < pn;
       pdec[t] = live ? __uint_as_float(word_of(gw, 2 * QM + 5 + t)) : 1.0f;
     }
+    wave_lds_sync();
+    if constexpr (PK_REGS) {
+#pragma unroll
+      for (int t = 0; t < QM; ++t)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+          for (int e = 0; e < E; ++e) pkr[t][j][e] = pk_lds[t][(16 * j + kb) * E + e];
+    }
   }
-  wave_lds_sync();
 
   // DEFER: replay the pending accepted prefix on one block in registers,
   // h <- fma(c_t, k_t, h * d_t) as the fold does, storing the boundary snapshot
   // after `boundary_len` tokens and the final state after n (kernels.py:1242-1324).
   // The final store is issued on every path (an unused one falls out of
-  // range) so the wait counts of the loads in flight do not depend on the row.
-  // The boundary snapshot's store, with its two LDS rounds, only runs on rows
-  // that have one (about one tile in seven at B=256): skipping the round trip
-  // elsewhere took the 48-layer deferred loop from 5.37-5.46 to 5.32 ms per
-  // step, which outweighs the stricter waits on the snapshot rows.
-  auto fold_block = [&](int rb, uint4 (&buf)[J], const float (&pc)[QM]) {
+  // range) so the wait counts of the loads in flight do not depend on the row;
+  // the boundary snapshot's only on rows that have one (about one tile in
+  // seven at B=256).
+  auto fold_block = [&](int rb, uint4 (&buf)[BR]) {
     if constexpr (DEFER) {
       const int seg = pstore_b ? pblen : 0;
       // FP32 values of the lane's chunks; the fold keeps them in FP32 across
       // the boundary snapshot and rounds only what it stores, as the fold does.
-      float h[J][E];
+      float h[BR][E];
 #pragma unroll
-      for (int j = 0; j < J; ++j) unpack16<S>(buf[j], h[j]);
+      for (int i = 0; i < BR; ++i) unpack16<S>(buf[i], h[i]);
       auto apply = [&](int lo, int hi) {
 #pragma unroll
         for (int t = 0; t < QM; ++t) {
           if (t >= lo && t < hi) {
-            const float d = pdec[t], c = pc[t];
+            const float d = pdec[t];
+            float c[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) c[g] = pc_lds[t][(rb & (HRB - 1)) * 16 + 4 * g + ij];
 #pragma unroll
             for (int j = 0; j < J; ++j) {
+              float kv[E];
 #pragma unroll
-              for (int e4 = 0; e4 < E; e4 += 4) {
-                const float4 kv = *reinterpret_cast<const float4 *>(&pk_lds[t][E * (4 * j + ls) + e4]);
-                h[j][e4 + 0] = __builtin_fmaf(c, kv.x, h[j][e4 + 0] * d);
-                h[j][e4 + 1] = __builtin_fmaf(c, kv.y, h[j][e4 + 1] * d);
-                h[j][e4 + 2] = __builtin_fmaf(c, kv.z, h[j][e4 + 2] * d);
-                h[j][e4 + 3] = __builtin_fmaf(c, kv.w, h[j][e4 + 3] * d);
+              for (int e = 0; e < E; ++e) {
+                if constexpr (PK_REGS)
+                  kv[e] = pkr[t][j][e];
+                else
+                  kv[e] = pk_lds[t][(16 * j + kb) * E + e];
               }
+#pragma unroll
+              for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < E; ++e) h[g * J + j][e] = __builtin_fmaf(c[g], kv[e], h[g * J + j][e] * d);
             }
           }
         }
       };
       auto store = [&](__amdgpu_buffer_rsrc_t r) {
-        if constexpr (NT) {
-          // Row runs, non-temporal: the folded chunks go back through LDS
-          // into the load layout (each lane writes the slots it read its
-          // operands from). Stores of 64-byte pieces of 16 rows ran slower,
-          // and non-temporal ones much slower: a synthetic twin of this
-          // launch's traffic took 224 us with the operand-layout stores and
-          // 192 us with whole-row non-temporal ones.
+        // Non-temporal row runs, as loaded (see the deferred rule in verify.hip).
 #pragma unroll
-          for (int g = 0; g < ROUNDS; ++g) {
+        for (int g = 0; g < 4; ++g)
 #pragma unroll
-            for (int j = g * JR; j < (g + 1) * JR; ++j)
-              *reinterpret_cast<uint4 *>(verify_stage[op_slot(j)]) = pack16<S>(h[j]);
-            wave_lds_sync();
-            // The round's row runs are read back first, then stored: each
-            // store's wait then holds back only the stores behind it.
-            uint4 x[JR];
-#pragma unroll
-            for (int j = 0; j < JR; ++j) x[j] = *reinterpret_cast<const uint4 *>(verify_stage[row_slot(g * JR + j)]);
-#pragma unroll
-            for (int j = 0; j < JR; ++j)
-              store_b128_settled<kPolicyNT>(__builtin_bit_cast(gdn_u32x4, x[j]), r, c_voff(g * JR + j),
-                                            c_soff(rb, g * JR + j));
-            wave_lds_sync();
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < J; ++j) {
-            const int vo = (4 * j + ls) * E < K ? lane_off + j * 64 : kOutOfRange;
-            store_b128_settled<0>(__builtin_bit_cast(gdn_u32x4, pack16<S>(h[j])), r, vo, rb * 16 * row_bytes);
-          }
-        }
+          for (int j = 0; j < J; ++j)
+            store_b128_settled<NT ? kPolicyNT : 0>(__builtin_bit_cast(gdn_u32x4, pack16<S>(h[g * J + j])), r,
+                                                   s_voff(j), s_soff(rb, g, j));
       };
       apply(0, seg);
       if (pstore_b) store(rbnd);
@@ -695,112 +769,72 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
       store(rfin);
       // The window is verified from the folded tile as stored.
 #pragma unroll
-      for (int j = 0; j < J; ++j) buf[j] = pack16<S>(h[j]);
+      for (int i = 0; i < BR; ++i) buf[i] = pack16<S>(h[i]);
     }
   };
 
-  if (a.l2norm) {
-    // kernels.py:645-648: x * rsqrt(sum(x*x) + 1e-6) for q and k, then q *= scale.
-    if (lane < NV) {
-      float ss = 0.0f;
-      for (int kk = 0; kk < KP; ++kk) ss += m_lds[lane][kk] * m_lds[lane][kk];
-      inv_lds[lane] = rsqrtf(ss + 1e-6f);
-    }
-    wave_lds_sync();
+  // ---- 5. pipelined S_0 . [k, q~] on the matrix cores, recurrence per half ----
+  auto gemv_block = [&](int rb, const uint4 (&src)[BR]) {
+    float y[CG];
 #pragma unroll
-    for (int p = 0; p < STAGE_PASSES; ++p) {
-      const int idx = p * kVerifyThreads + lane;
-      const int vid = idx / C4, kk = (idx - vid * C4) * 4;
-      if (vid < NV) {
-        const bool is_q = vid >= QM;
-        const int t = is_q ? vid - QM : vid;
-        const bool wr = !is_q && key_writer && ((valid_mask >> t) & 1u) && kk < K;
-        const int64_t base = int64_t(b) * a.key_rs + int64_t(key_head) * a.key_hs + int64_t(t) * a.key_ts + kk;
+    for (int g = 0; g < 4; ++g) {
+      f32x4 acc[CG];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x = m_lds[vid][kk + e] * inv_lds[vid];
-          m_lds[vid][kk + e] = x * (is_q ? a.scale : 1.0f);
-          if (wr) st_f32_or<A>(a.key, base + e, key_f32, x);
+      for (int cg = 0; cg < CG; ++cg) acc[cg] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const float x = chunk_elem<S>(src[g * J + j], e);
+#pragma unroll
+          for (int cg = 0; cg < CG; ++cg)
+            acc[cg] = __builtin_amdgcn_mfma_f32_4x4x1f32(x, m[cg][j][e], acc[cg], 0, 0, 0);
         }
+      // Rows 4g .. 4g+3: every copy holds the sums; copy g keeps them.
+#pragma unroll
+      for (int cg = 0; cg < CG; ++cg) {
+        const float r = reduce_rows(acc[cg]);
+        y[cg] = g == 0 || bq == g ? r : y[cg];
       }
     }
-    wave_lds_sync();
-  }
-
-  // ---- 5. Gram matrix k_s . m_j (8 lanes per dot product, DPP sum) ----
-  {
-    const int j8 = lane & 7;
-    for (int d0 = 0; d0 < QM * NV; d0 += kVerifyThreads / 8) {
-      const int d = d0 + (lane >> 3);
-      const int s = d / NV, j = d - (d / NV) * NV;
-      float part = 0.0f;
-      if (d < QM * NV) {
-        constexpr int GL = KP / 8;
+    const int row = (rb & (HRB - 1)) * 16 + 4 * bq + q16;
 #pragma unroll
-        for (int e = 0; e < GL; ++e) part += m_lds[s][j8 * GL + e] * m_lds[j][j8 * GL + e];
-      }
-      part = dpp_sum8(part);
-      if (d < QM * NV && j8 == 0) gram_lds[s][j] = part;
-    }
-  }
-  // B operands come from LDS per chunk group inside every block: keeping all of
-  // them in registers would cost the occupancy the load pipeline needs. Lanes
-  // of columns >= NV read some valid row: those columns of D are never used.
-  const bool col_live = li < NV;
-  const int brow = li & (NV - 1);
-
-  // ---- 6. pipelined S_0 . [k, q~] on the matrix cores, recurrence per half ----
-  auto gemv_block = [&](int rb, const uint4 (&src)[J]) {
-    asm volatile("" ::: "memory");  // re-read the B operands for every block
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      float bop[E];
-#pragma unroll
-      for (int e = 0; e < E; ++e) bop[e] = m_lds[brow][E * (4 * j + ls) + e];
-#pragma unroll
-      for (int e = 0; e < E; ++e)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(chunk_elem<S>(src[j], e), bop[e], acc, 0, 0, 0);
-    }
-    if (col_live) {
-      const int rr = (rb & 3) * 16 + 4 * ls;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) d_lds[rr + r][li] = acc[r];
-    }
+    for (int cg = 0; cg < CG; ++cg)
+      if (NV % 4 == 0 || 4 * cg + ij < NV) d_lds[row][4 * cg + ij] = y[cg];
   };
   // Outputs and corrections go out through buffer stores that are issued for
   // every token and lane (an invalid one gets an out-of-range offset and is
   // dropped): a store skipped on some path would make the wait counts of the
   // loads still in flight assume it, and drain the pipeline at the next block.
-  const bool out_f32 = a.out_f32 != 0;
-  const __amdgpu_buffer_rsrc_t rout = make_rsrc(a.out, (bos * a.out_ts + out_base) * (out_f32 ? 4 : AS));
+  const bool out_f32 = z->out_f32 != 0;
+  const __amdgpu_buffer_rsrc_t rout = make_rsrc(z->out, (bos * z->out_ts + out_base) * (out_f32 ? 4 : AS));
   const __amdgpu_buffer_rsrc_t rcorr =
-      make_rsrc(a.corr, (int64_t(b) * a.corr_rs + int64_t(hv) * a.corr_hs + row0) * 4);
+      make_rsrc(z->corr, (int64_t(b) * z->corr_rs + int64_t(hv) * z->corr_hs + row0) * 4);
   float res_c[2][QM], res_o[2][QM];  // corrections and outputs of the lane's row in each half
   auto emit = [&](int half) {
     const int lrow = half * 64 + lane;
-    int row_ok = row0 + lrow < V;
+    int row_ok = (row0 + lrow < V) & (lane < HALF);
     asm volatile("" : "+v"(row_ok));  // per-lane offsets below, not branches
 #pragma unroll
     for (int t = 0; t < QM; ++t) {
       const bool st = ((valid_mask >> t) & 1u) && row_ok;
-      const int oel = t * int(a.out_ts) + lrow;
+      const int oel = t * int(z->out_ts) + lrow;
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(res_o[half][t]), rout,
                                             st && out_f32 ? oel * 4 : kOutOfRange, 0, 0);
       if constexpr (sizeof(A) == 2)
         __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, from_f32<A>(res_o[half][t])), rout,
                                               st && !out_f32 ? oel * AS : kOutOfRange, 0, 0);
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(res_c[half][t]), rcorr,
-                                            st && rec_ok ? (t * a.corr_ts + lrow) * 4 : kOutOfRange, 0, 0);
+                                            st && rec_ok ? (t * z->corr_ts + lrow) * 4 : kOutOfRange, 0, 0);
     }
   };
   auto recurrence = [&](int half) {
-    wave_lds_sync();  // d_lds (and, on the first half, gram_lds) complete
+    wave_lds_sync();  // d_lds complete
     float u[QM], wq[QM];
 #pragma unroll
     for (int t = 0; t < QM; ++t) {
-      u[t] = d_lds[lane][t];
-      wq[t] = d_lds[lane][QM + t];
+      u[t] = d_lds[lane & (HALF - 1)][t];
+      wq[t] = d_lds[lane & (HALF - 1)][QM + t];
     }
 #pragma unroll
     for (int t = 0; t < QM; ++t) {
@@ -809,9 +843,9 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
       const float c = tv ? (vv[half][t] - d * u[t]) * bet[t] : 0.0f;
       if (tv) {
 #pragma unroll
-        for (int j = t + 1; j < QM; ++j) u[j] = __builtin_fmaf(c, gram_lds[t][j], d * u[j]);
+        for (int j = t + 1; j < QM; ++j) u[j] = __builtin_fmaf(c, dot(t, j), d * u[j]);
 #pragma unroll
-        for (int j = t; j < QM; ++j) wq[j] = __builtin_fmaf(c, gram_lds[t][QM + j], d * wq[j]);
+        for (int j = t; j < QM; ++j) wq[j] = __builtin_fmaf(c, dot(t, QM + j), d * wq[j]);
       }
       res_c[half][t] = c;
       res_o[half][t] = wq[t];
@@ -821,39 +855,31 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
   };
 #pragma unroll
   for (int rb = 0; rb < NRB; rb += 2) {
-    if constexpr (NT && !DEFER) {
-      // Once a block sits in LDS its registers take the block after next:
-      // those loads issue before the block's last read-back and its matrix
-      // work.
-      uint4 op[J];
-      auto stage_block = [&](int next, uint4 (&buf)[J], float (&pc)[QM]) {
-#pragma unroll
-        for (int g = 0; g < ROUNDS; ++g) {
-          stage_write(buf, g);
-          if (g + 1 == ROUNDS && next < NRB) load_block(next, buf, pc);
-          wave_lds_sync();
-          stage_read(op, g);
-          wave_lds_sync();
-        }
-      };
-      stage_block(rb + 2, bufA, pcA);
-      gemv_block(rb, op);
-      stage_block(rb + 3, bufB, pcB);
-      gemv_block(rb + 1, op);
-    } else {
-      transpose(bufA);
-      fold_block(rb, bufA, pcA);
-      gemv_block(rb, bufA);
-      if (rb + 2 < NRB) load_block(rb + 2, bufA, pcA);
-      transpose(bufB);
-      fold_block(rb + 1, bufB, pcB);
+    fold_block(rb, bufA);
+    gemv_block(rb, bufA);
+    if (rb + 2 < NRB) load_block(rb + 2, bufA);
+    if constexpr (NRB > 1) {
+      fold_block(rb + 1, bufB);
       gemv_block(rb + 1, bufB);
-      if (rb + 3 < NRB) load_block(rb + 3, bufB, pcB);
+      if (rb + 3 < NRB) load_block(rb + 3, bufB);
     }
-    if (NRB == 8 && rb + 2 == NRB / 2) load_v(1);  // a half tile has no second half
+    if (NRB == 8 && rb + 2 == NRB / 2) load_v(1);  // smaller tiles have no second half
     // Every half runs its recurrence, also one past V (its rows store nothing):
     // skipping it would be a path without its stores.
-    if ((rb + 2) % 4 == 0) recurrence((rb + 2) / 4 - 1);
+    if (HRB < 4 || (rb + 2) % 4 == 0) recurrence(HRB < 4 ? 0 : (rb + 2) / 4 - 1);
+  }
+  };
+  if constexpr (TILE == 128) {
+    // Long tiles: the rest's arguments are read where they are used, not with
+    // the others at the kernel's start, from where they were held in spilled
+    // registers (12 layers of 64 rows: verify + commit 909 against 922 us).
+    // Short tiles are a chain of latencies, and the reads lengthened it (24
+    // layers of 16 rows: 534 against 512 us).
+    const auto *z = (const __attribute__((address_space(4))) VerifyArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(z));
+    rest(z);
+  } else {
+    rest(&a);
   }
 }
 
@@ -864,76 +890,86 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 4
 // still be there. Reading the earlier part non-temporally keeps it from
 // evicting that part (and the non-temporal reads run faster): the host sets
 // nt_rows so that the ordinary reads cover the last `retain` bytes.
-template <typename S, typename A, int J, int QM, bool DEFER>
-__global__ __launch_bounds__(kVerifyThreads) void verify_kernel(VerifyArgs a) {
-  __shared__ VerifyLds<QM, 4 * Chunk<S>::E * J, J, DEFER> lds;
+// Long tiles keep three waves per SIMD (168 registers): left free, Q = 8 takes
+// 184 registers and two waves (B=256 step 306 against 287 us); four waves
+// spill (318 us).
+template <typename S, typename A, int J, int QM, bool DEFER, int TILE>
+__global__ __launch_bounds__(kVerifyThreads, TILE == 128 ? 3 : 1) void verify_kernel(VerifyArgs a) {
+  __shared__ VerifyLds<QM, 16 * Chunk<S>::E * J, DEFER, TILE> lds;
+  warm_kernel_args<int(sizeof(VerifyArgs))>();
   if (DEFER || int(blockIdx.y) < a.nt_rows)  // the deferred verify: every row (see verify.hip)
-    verify_wave<S, A, J, QM, DEFER, true>(a, lds);
+    verify_wave<S, A, J, QM, DEFER, true, TILE>(a, lds);
   else
-    verify_wave<S, A, J, QM, DEFER, false>(a, lds);
+    verify_wave<S, A, J, QM, DEFER, false, TILE>(a, lds);
 }
 
 // Launch for one state type; defined per state type in verify_<state>.hip.
 template <typename S>
-void launch_verify_state(int act_dt, int j, int qm, bool deferred, dim3 grid, hipStream_t s, const VerifyArgs &a);
+void launch_verify_state(int act_dt, int j, int tile, int qm, bool deferred, dim3 grid, hipStream_t s,
+                         const VerifyArgs &a);
 
-template <typename S, typename A, int J, bool DEFER>
+template <typename S, typename A, int J, bool DEFER, int TILE>
 static void launch_verify_q(int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
-  // The staging block only for launches with non-temporal rows (it costs
-  // occupancy otherwise).
-  const unsigned lds = DEFER || a.nt_rows > 0 ? unsigned(verify_stage_bytes(J)) : 0u;
+  const dim3 wg(kVerifyThreads);
   switch (qm) {
-    case 1: hipLaunchKernelGGL((verify_kernel<S, A, J, 1, DEFER>), grid, dim3(kVerifyThreads), lds, s, a); break;
-    case 2: hipLaunchKernelGGL((verify_kernel<S, A, J, 2, DEFER>), grid, dim3(kVerifyThreads), lds, s, a); break;
-    case 4: hipLaunchKernelGGL((verify_kernel<S, A, J, 4, DEFER>), grid, dim3(kVerifyThreads), lds, s, a); break;
-    default: hipLaunchKernelGGL((verify_kernel<S, A, J, 8, DEFER>), grid, dim3(kVerifyThreads), lds, s, a); break;
+    case 1: hipLaunchKernelGGL((verify_kernel<S, A, J, 1, DEFER, TILE>), grid, wg, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((verify_kernel<S, A, J, 2, DEFER, TILE>), grid, wg, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((verify_kernel<S, A, J, 4, DEFER, TILE>), grid, wg, 0, s, a); break;
+    default: hipLaunchKernelGGL((verify_kernel<S, A, J, 8, DEFER, TILE>), grid, wg, 0, s, a); break;
   }
 }
 
-// J: 16-byte chunks per lane per row, KP = 4 * E * J <= 256, so J <= 16 for
-// f32 state and J <= 8 for 16-bit state.
+template <typename S, typename A, int J, bool DEFER>
+static void launch_verify_tile(int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
+  switch (tile) {
+    case 16: launch_verify_q<S, A, J, DEFER, 16>(qm, grid, s, a); break;
+    case 64: launch_verify_q<S, A, J, DEFER, 64>(qm, grid, s, a); break;
+    default: launch_verify_q<S, A, J, DEFER, DEFER ? 32 : 128>(qm, grid, s, a); break;
+  }
+}
+
+// J: 16-byte chunks per lane per row, KP = 16 * E * J <= 256, so J <= 4 for
+// f32 state and J <= 2 for 16-bit state.
 template <typename S, typename A, bool DEFER>
-static void launch_verify_j(int j, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
+static void launch_verify_j(int j, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
   switch (j) {
-    case 1: launch_verify_q<S, A, 1, DEFER>(qm, grid, s, a); break;
-    case 2: launch_verify_q<S, A, 2, DEFER>(qm, grid, s, a); break;
-    case 4: launch_verify_q<S, A, 4, DEFER>(qm, grid, s, a); break;
-    case 8: launch_verify_q<S, A, 8, DEFER>(qm, grid, s, a); break;
+    case 1: launch_verify_tile<S, A, 1, DEFER>(tile, qm, grid, s, a); break;
+    case 2: launch_verify_tile<S, A, 2, DEFER>(tile, qm, grid, s, a); break;
     default:
-      if constexpr (Chunk<S>::E == 4) launch_verify_q<S, A, 16, DEFER>(qm, grid, s, a);
+      if constexpr (Chunk<S>::E == 4) launch_verify_tile<S, A, 4, DEFER>(tile, qm, grid, s, a);
       break;
   }
 }
 
 template <typename S, bool DEFER>
-static void launch_verify_act(int act_dt, int j, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
+static void launch_verify_act(int act_dt, int j, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
   switch (act_dt) {
-    case GDN_DT_BF16: launch_verify_j<S, bf16, DEFER>(j, qm, grid, s, a); break;
-    case GDN_DT_F16: launch_verify_j<S, f16, DEFER>(j, qm, grid, s, a); break;
-    default: launch_verify_j<S, float, DEFER>(j, qm, grid, s, a); break;
+    case GDN_DT_BF16: launch_verify_j<S, bf16, DEFER>(j, tile, qm, grid, s, a); break;
+    case GDN_DT_F16: launch_verify_j<S, f16, DEFER>(j, tile, qm, grid, s, a); break;
+    default: launch_verify_j<S, float, DEFER>(j, tile, qm, grid, s, a); break;
   }
 }
 
 // The deferred-commit kernels of each state type live in a translation unit of
 // their own (verify_<state>_deferred.hip), so the halves compile in parallel.
 template <typename S>
-void launch_verify_deferred(int act_dt, int j, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a);
+void launch_verify_deferred(int act_dt, int j, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a);
 
 #define GDN_DEFINE_VERIFY_LAUNCH(STATE)                                                                \
   template <>                                                                                          \
-  void launch_verify_state<STATE>(int act_dt, int j, int qm, bool deferred, dim3 grid, hipStream_t s, \
+  void launch_verify_state<STATE>(int act_dt, int j, int tile, int qm, bool deferred, dim3 grid, hipStream_t s, \
                                   const VerifyArgs &a) {                                               \
     if (deferred)                                                                                      \
-      launch_verify_deferred<STATE>(act_dt, j, qm, grid, s, a);                                        \
+      launch_verify_deferred<STATE>(act_dt, j, tile, qm, grid, s, a);                                        \
     else                                                                                               \
-      launch_verify_act<STATE, false>(act_dt, j, qm, grid, s, a);                                      \
+      launch_verify_act<STATE, false>(act_dt, j, tile, qm, grid, s, a);                                      \
   }
 
 #define GDN_DEFINE_VERIFY_DEFERRED_LAUNCH(STATE)                                                         \
   template <>                                                                                            \
-  void launch_verify_deferred<STATE>(int act_dt, int j, int qm, dim3 grid, hipStream_t s,                \
+  void launch_verify_deferred<STATE>(int act_dt, int j, int tile, int qm, dim3 grid, hipStream_t s,                \
                                      const VerifyArgs &a) {                                              \
-    launch_verify_act<STATE, true>(act_dt, j, qm, grid, s, a);                                           \
+    launch_verify_act<STATE, true>(act_dt, j, tile, qm, grid, s, a);                                           \
   }
 
 }  // namespace gdn

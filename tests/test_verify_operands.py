@@ -1,0 +1,87 @@
+"""The verify kernel's lane arithmetic (csrc/verify_kernel.cuh), restated on the
+CPU: `reduce_rows` over the 16 blocks of a 4x4x1 matrix instruction, the loads'
+cover of a 16-row block, `udiv`, and the runs of 16-bit elements that start in
+either half of a dword (`load_run`)."""
+
+import random
+
+import pytest
+
+
+def _swap32(x, y):
+    return x[:32] + y[:32], x[32:] + y[32:]
+
+
+def _swap16(x, y):
+    rows = lambda a: [a[16 * i:16 * i + 16] for i in range(4)]  # noqa: E731
+    a, b = rows(x), rows(y)
+    return a[0] + b[0] + a[2] + b[2], a[1] + b[1] + a[3] + b[3]
+
+
+def _add(p):
+    return [a + b for a, b in zip(*p)]
+
+
+def _ror(x, n):
+    return [x[16 * (i // 16) + (i % 16 - n) % 16] for i in range(64)]
+
+
+def test_reduce_rows_sums_the_blocks():
+    rng = random.Random(1)
+    acc = [[rng.randrange(1 << 20) for _ in range(64)] for _ in range(4)]  # register r, lane 4*block + column
+    x = _add(_swap16(_add(_swap32(acc[0], acc[2])), _add(_swap32(acc[1], acc[3]))))
+    x = _add((x, _ror(x, 8)))
+    x = _add((x, _ror(x, 4)))
+    for lane in range(64):
+        r, col = lane >> 4, lane & 3
+        assert x[lane] == sum(acc[r][4 * kb + col] for kb in range(16))
+
+
+@pytest.mark.parametrize("J", [1, 2, 4])
+def test_block_loads_are_whole_row_runs(J):
+    """Register g*J + j of lane 4*kb + ij holds chunk 16j + kb of row 4g + ij: each
+    chunk once, every load four runs of 16 consecutive chunks."""
+    seen = []
+    for g in range(4):
+        for j in range(J):
+            at = [(4 * g + (lane & 3), 16 * j + (lane >> 2)) for lane in range(64)]
+            assert sorted(at) == [(4 * g + r, 16 * j + c) for r in range(4) for c in range(16)]
+            seen += at
+    assert sorted(seen) == [(r, c) for r in range(16) for c in range(16 * J)]
+
+
+def test_udiv_is_exact():
+    rng = random.Random(2)
+    ds = [1, 2, 3, 5, 7, 12, 31, 64, 1000, 65535, 65537, (1 << 31) - 1, 1 << 31, (1 << 32) - 1]
+    ds += [rng.randrange(1, 1 << rng.randrange(1, 33)) for _ in range(300)]
+    for d in ds:
+        m = 0xFFFFFFFF // d
+        xs = {0, 1, d - 1, d, d + 1, 2 * d - 1, 2 * d, 0x7FFFFFFF, 0xFFFFFFFF, (0xFFFFFFFF // d) * d, (0xFFFFFFFF // d) * d - 1}
+        xs |= {rng.randrange(1 << 32) for _ in range(50)}
+        for x in xs:
+            if not 0 <= x < 1 << 32:
+                continue
+            q = (x * m) >> 32
+            q += x - q * d >= d
+            assert q == x // d, (x, d)
+
+
+@pytest.mark.parametrize("N", [4, 8])
+@pytest.mark.parametrize("first", range(8))
+def test_runs_of_16_bit_elements(N, first):
+    """A run from any element: the dwords read hold elements of the run only,
+    and the funnel shift lines them up."""
+    elems = [0x1000 + i for i in range(32)]
+    words = [elems[2 * i] | elems[2 * i + 1] << 16 for i in range(16)]
+    off = first * 2
+    odd = off & 2
+    at = off // 4
+    got = words[at:at + N // 2] + [words[at + N // 2] if odd else 0]
+    touched = range(at, at + N // 2 + (1 if odd else 0))
+    assert all(2 * w + 1 >= first and 2 * w < first + N for w in touched)
+    sh = 16 if odd else 0
+    out = []
+    for i in range(N // 2):
+        u = (((got[i + 1] << 32) | got[i]) >> sh) & 0xFFFFFFFF
+        out += [u & 0xFFFF, u >> 16]
+    assert out == elems[first:first + N]
