@@ -9,8 +9,10 @@
 namespace gdn {
 
 // ----------------------------------------------------------------------------
-// Element conversions. bf16 <-> f32 are bit operations (round-to-nearest-even on
-// the way down, NaN kept quiet); f16 uses the hardware conversion.
+// Element conversions. bf16 -> f32 is a shift; f32 -> bf16 is gfx950's packed
+// conversion (v_cvt_pk_bf16_f32: round to nearest even, NaN kept quiet; all
+// 2^32 inputs give the bits of the shift-and-add form, which took six vector
+// instructions per element). f16 uses the hardware conversion.
 // ----------------------------------------------------------------------------
 struct bf16 {
   uint16_t bits;
@@ -27,10 +29,7 @@ template <>
 __device__ __forceinline__ float from_f32<float>(float x) { return x; }
 template <>
 __device__ __forceinline__ bf16 from_f32<bf16>(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return bf16{uint16_t((u >> 16) | 0x0040u)};
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return bf16{uint16_t(u >> 16)};
+  return bf16{__builtin_bit_cast(uint16_t, static_cast<__bf16>(x))};
 }
 // The conversion starts from the rounded FP32 value: left to itself the
 // compiler folds a multiply-add that produced x into the conversion (one
@@ -175,10 +174,12 @@ __device__ __forceinline__ uint4 pack16<float>(const float *in) {
 }
 template <>
 __device__ __forceinline__ uint4 pack16<bf16>(const float *in) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   uint32_t w[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    w[i] = uint32_t(from_f32<bf16>(in[2 * i]).bits) | (uint32_t(from_f32<bf16>(in[2 * i + 1]).bits) << 16);
+    w[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{in[2 * i], in[2 * i + 1]}), bf16x2));
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 template <>
