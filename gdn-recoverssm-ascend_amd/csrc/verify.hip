@@ -12,24 +12,26 @@ static bool float_dt_ok(int32_t dt) { return dt == GDN_DT_F32 || dt == GDN_DT_BF
 // block and 9 us with eight, so a launch that leaves the chip's 1024 SIMDs idle
 // takes short tiles; a wave's own reads of q, k, gates and its Gram matrix
 // repeat per tile, so a launch bound by memory takes long ones. Times in us of
-// 48 layers' worth of K = V = 128 FP32 pages, Q = 4, HV = 32, tiles of 16 / 64 /
-// 128 rows: 1 row 5.4 / 7.5 / 11.2, 4 rows 5.9 / 7.6 / 11.2, 8 rows 9.1 / 8.6 /
-// 12.0, 16 rows 13.8 / 12.5 / 13.9, 24 rows 18.4 / 17.2 / 16.9, 32 rows 22.7 /
-// 22.0 / 21.0, 64 rows 38 / 36 / 35; BF16 pages: 32 rows 21 / 14.7 / 15.6, 64
-// rows 37 / 23.7 / 23.9. At Q = 1 a wave has half the columns and a quarter of
-// the outputs, and 16-row tiles stay ahead up to 64 rows (16 rows 10.2 / 11.8 /
-// 11.2, 64 rows 28.1 / 31.7 / 31.2, 128 rows 51 / 53 / 52).
+// one layer of several with K = V = 128 FP32 pages, Q = 4, HV = 32, tiles of 16 /
+// 64 / 128 rows: 1 row 5.4 / 7.5 / 11.2, 4 rows 5.9 / 7.6 / 11.2, 8 rows 9.1 /
+// 8.6 / 12.0, 16 rows 13.8 / 12.5 / 13.9; 64 / 128 rows: 24 rows 17.0 / 17.9, 40
+// rows (2560 waves of 64) 24.1 / 24.3, 48 rows 28.3 / 27.1, gated 37 rows 24.2 /
+// 25.2, BF16 pages 32 rows 14.7 / 15.6, 48 rows 20.8 / 20.2. At Q = 8 a wave's own
+// reads and Gram matrix are four times as large: 16 rows 16.5 / 19.9, 24 rows
+// 24.2 / 22.1. At Q = 1 they are a fraction, and 16-row tiles stay ahead up to
+// 64 rows (16 / 64 / 128: 16 rows 10.2 / 11.8 / 11.2, 64 rows 28.1 / 31.7 / 31.2,
+// 128 rows 51 / 53 / 52).
 //
 // The deferred verify also writes the tile back, and a launch's time steps with
 // its rounds of resident waves (3 per SIMD, 3072): the smallest tile whose
 // waves fit one round, else 32 rows (tiles of 16 / 32 / 64 rows: 1 row 6.8 /
 // 8.4 / 10.9, 8 rows 12.1 / 13.2 / 14.2, 16 rows 18.6 / 18.1 / 18.4, 32 rows
 // 35 / 32.6 / 30.6, 64 rows 60 / 58 / 61, 128 rows 110 / 105 / 105).
-static int verify_tile(int64_t rows, int64_t value_heads, int64_t V, int64_t row_bytes, int qm, bool deferred) {
+static int verify_tile(int64_t rows, int64_t value_heads, int64_t V, int qm, bool deferred) {
   auto waves = [&](int tile) { return rows * value_heads * ((V + tile - 1) / tile); };
   if (deferred) return waves(16) <= 3072 ? 16 : waves(32) <= 3072 ? 32 : waves(64) <= 3072 ? 64 : 32;
   if (waves(16) <= (qm == 1 ? 16384 : 1280)) return 16;
-  return rows * value_heads * V * row_bytes <= (int64_t(48) << 20) ? 64 : 128;
+  return waves(64) <= (qm == 8 ? 1024 : 2560) ? 64 : 128;
 }
 
 static bool fits_i32(int64_t x) { return x >= INT32_MIN && x <= INT32_MAX; }
@@ -228,7 +230,7 @@ static int verify_impl(const void *q, const void *k, const void *v, const void *
   int j = 1;
   while (16 * E * j < K) j *= 2;
   const int qm = Q <= 1 ? 1 : Q <= 2 ? 2 : Q <= 4 ? 4 : 8;
-  const int tile = verify_tile(rows, value_heads, V, K * (E == 4 ? 4 : 2), qm, pending != nullptr);
+  const int tile = verify_tile(rows, value_heads, V, qm, pending != nullptr);
   a.NVT = int32_t((V + tile - 1) / tile);
   a.nvt_magic = udiv_magic(uint32_t(a.NVT));
   if (int64_t(a.NVT) * value_heads > 0x7fffffffLL) {

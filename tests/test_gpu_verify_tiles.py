@@ -29,11 +29,11 @@ def test_value_dims_around_the_tiles(dev, V, state):
     _run_and_check(_problem(3, 1, 2, 64, V, 4, qlens=[4, 1, 3], seed=V, state_dtype=state), dev)
 
 
-@pytest.mark.parametrize("B,HV,V,Q", [(5, 32, 128, 4), (6, 32, 120, 4), (20, 32, 72, 3), (26, 32, 130, 4),
+@pytest.mark.parametrize("B,HV,V,Q", [(5, 32, 128, 4), (6, 32, 120, 4), (20, 32, 72, 3), (26, 32, 130, 4), (28, 32, 130, 4),
                                       (26, 32, 136, 8), (65, 32, 128, 1), (66, 32, 136, 1), (30, 32, 128, 2)])
 def test_batches_around_each_line(dev, B, HV, V, Q):
-    # 16 -> 64 rows past 1280 waves of 16, 64 -> 128 past 48 MiB of state; Q = 1
-    # keeps 16 rows to 16384 waves.
+    # 16 -> 64 rows past 1280 waves of 16, 64 -> 128 past 2560 waves of 64 (Q = 8:
+    # 1024); Q = 1 keeps 16 rows to 16384 waves.
     _run_and_check(_problem(B, 4, HV, 128, V, Q, seed=B + V, null_rows=(1,)), dev)
 
 
