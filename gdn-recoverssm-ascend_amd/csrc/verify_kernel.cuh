@@ -603,11 +603,14 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       if constexpr (QM % 4 != 0) {
-        float xk[E], xq[E];
-        unpack_run<A, E>(raw_k[cg][j], xk);
-        unpack_run<A, E>(raw_q[cg][j], xq);
+        // One of the two was read out of range, as zeros. Their words are ORed:
+        // a sum would lose the sign of a zero, and the key record holds the
+        // key's own bits.
+        RawRun<A, E> x = raw_k[cg][j];
 #pragma unroll
-        for (int e = 0; e < E; ++e) m[cg][j][e] = xk[e] + xq[e];
+        for (int i = 0; i < int(sizeof(x.w) / 4); ++i) x.w[i] |= raw_q[cg][j].w[i];
+        if constexpr (sizeof(A) == 2) x.sh = 4 * cg + ij >= QM ? raw_q[cg][j].sh : x.sh;
+        unpack_run<A, E>(x, m[cg][j]);
       } else {
         unpack_run<A, E>(4 * cg < QM ? raw_k[cg][j] : raw_q[cg][j], m[cg][j]);
       }
