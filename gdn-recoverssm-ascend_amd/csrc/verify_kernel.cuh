@@ -293,6 +293,13 @@ struct __align__(16) VerifyLds {
   float pc[DEFER ? QM : 1][DEFER ? HALF : 1];              // and its corrections of the tile's rows
 };
 
+// Rows of a block: 16, or 8 where the two block buffers (32J registers a lane at
+// 16 rows) and the 64 registers of B operands of FP32 pages of K > 128 at Q > 4
+// would take a wave all its SIMD's registers: at 16 rows that kernel had one
+// wave per SIMD, or spilled (K = 256, Q = 8, 32 heads, 64 rows: 143 us held to
+// three waves, 69 to two, 65 with blocks of 8 rows).
+__host__ __device__ constexpr int verify_block_rows(int e, int j, int qm) { return e == 4 && j == 4 && qm == 8 ? 8 : 16; }
+
 template <typename S, typename A, int J, int QM, bool DEFER, bool NT, int TILE>
 __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 16 * Chunk<S>::E * J, DEFER, TILE> &L) {
   static_assert(!DEFER || TILE <= 64, "the pending corrections cover one half tile");
@@ -301,9 +308,11 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
   constexpr int NV = 2 * QM;           // columns: k_0 .. k_{QM-1}, q~_0 .. q~_{QM-1}
   constexpr int CG = (NV + 3) / 4;     // groups of 4 columns
   constexpr int CGK = (QM + 3) / 4;    // column groups that hold a k
-  constexpr int NRB = TILE / 16;       // 16-row blocks per tile
+  constexpr int BROWS = verify_block_rows(E, J, QM);
+  constexpr int BG = BROWS / 4;        // 4-row groups of a block
+  constexpr int NRB = TILE / BROWS;    // blocks per tile
   constexpr int HALF = TILE < 64 ? TILE : 64;  // rows of one recurrence (one per lane)
-  constexpr int HRB = HALF / 16;
+  constexpr int HRB = HALF / BROWS;
   auto &d_lds = L.d;
   auto &pk_lds = L.pk;
   auto &pc_lds = L.pc;
@@ -541,16 +550,16 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
   // here became a 64-bit multiply-add whose unused high addend was a register
   // with a load in flight, and waiting for it held back the first state loads.
   const int lane_off = int(__umul24(unsigned(ij), unsigned(row_bytes))) + kb * 16;
-  constexpr int BR = 4 * J;  // registers (16-byte chunks per lane) of a block
+  constexpr int BR = BG * J;  // 16-byte chunks per lane of a block
   auto s_voff = [&](int j) { return (16 * j + kb) * E < K ? lane_off : kOutOfRange; };
-  auto s_soff = [&](int rb, int g, int j) { return (rb * 16 + 4 * g) * row_bytes + j * 256; };
+  auto s_soff = [&](int rb, int g, int j) { return (rb * BROWS + 4 * g) * row_bytes + j * 256; };
   // One form for every K, and every block is loaded (blocks past V read as
   // zero): a conditional load would leave a path on which it was not issued,
   // and the wait counts of every later MFMA would have to assume that path,
   // draining the pipeline at each block.
   auto load_block = [&](int rb, uint4 (&dst)[BR]) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < BG; ++g)
 #pragma unroll
       for (int j = 0; j < J; ++j)
         dst[g * J + j] = __builtin_bit_cast(
@@ -736,9 +745,9 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
         for (int t = 0; t < QM; ++t) {
           if (t >= lo && t < hi) {
             const float d = pdec[t];
-            float c[4];
+            float c[BG];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) c[g] = pc_lds[t][(rb & (HRB - 1)) * 16 + 4 * g + ij];
+            for (int g = 0; g < BG; ++g) c[g] = pc_lds[t][(rb & (HRB - 1)) * BROWS + 4 * g + ij];
 #pragma unroll
             for (int j = 0; j < J; ++j) {
               float kv[E];
@@ -750,7 +759,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
                   kv[e] = pk_lds[t][(16 * j + kb) * E + e];
               }
 #pragma unroll
-              for (int g = 0; g < 4; ++g)
+              for (int g = 0; g < BG; ++g)
 #pragma unroll
                 for (int e = 0; e < E; ++e) h[g * J + j][e] = __builtin_fmaf(c[g], kv[e], h[g * J + j][e] * d);
             }
@@ -760,7 +769,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
       auto store = [&](__amdgpu_buffer_rsrc_t r) {
         // Non-temporal row runs, as loaded (see the deferred rule in verify.hip).
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int g = 0; g < BG; ++g)
 #pragma unroll
           for (int j = 0; j < J; ++j)
             store_b128_settled<NT ? kPolicyNT : 0>(__builtin_bit_cast(gdn_u32x4, pack16<S>(h[g * J + j])), r,
@@ -780,7 +789,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
   auto gemv_block = [&](int rb, const uint4 (&src)[BR]) {
     float y[CG];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < BG; ++g) {
       f32x4 acc[CG];
 #pragma unroll
       for (int cg = 0; cg < CG; ++cg) acc[cg] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -800,10 +809,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
         y[cg] = g == 0 || bq == g ? r : y[cg];
       }
     }
-    const int row = (rb & (HRB - 1)) * 16 + 4 * bq + q16;
+    const int row = (rb & (HRB - 1)) * BROWS + 4 * bq + q16;
 #pragma unroll
     for (int cg = 0; cg < CG; ++cg)
-      if (NV % 4 == 0 || 4 * cg + ij < NV) d_lds[row][4 * cg + ij] = y[cg];
+      if ((BG == 4 || bq < BG) && (NV % 4 == 0 || 4 * cg + ij < NV)) d_lds[row][4 * cg + ij] = y[cg];
   };
   // Outputs and corrections go out through buffer stores that are issued for
   // every token and lane (an invalid one gets an out-of-range offset and is
@@ -866,10 +875,11 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
       gemv_block(rb + 1, bufB);
       if (rb + 3 < NRB) load_block(rb + 3, bufB);
     }
-    if (NRB == 8 && rb + 2 == NRB / 2) load_v(1);  // smaller tiles have no second half
+    if (TILE == 128 && rb + 2 == NRB / 2) load_v(1);  // smaller tiles have no second half
     // Every half runs its recurrence, also one past V (its rows store nothing):
     // skipping it would be a path without its stores.
-    if (HRB < 4 || (rb + 2) % 4 == 0) recurrence(HRB < 4 ? 0 : (rb + 2) / 4 - 1);
+    constexpr int PASS = HRB < 2 ? 2 : HRB;  // blocks of a half, taken two at a time
+    if ((rb + 2) % PASS == 0) recurrence((rb + 2) / PASS - 1);
   }
   };
   if constexpr (TILE == 128) {
@@ -893,11 +903,19 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
 // still be there. Reading the earlier part non-temporally keeps it from
 // evicting that part (and the non-temporal reads run faster): the host sets
 // nt_rows so that the ordinary reads cover the last `retain` bytes.
-// Long tiles keep three waves per SIMD (168 registers): left free, Q = 8 takes
-// 184 registers and two waves (B=256 step 306 against 287 us); four waves
-// spill (318 us).
+// Long tiles keep three waves per SIMD (168 registers) where they fit: left
+// free, Q = 8 at K = 128 takes 184 registers and two waves (B=256 step 306
+// against 287 us); four waves spill (318 us). They fit where the two block
+// buffers and the B operands take at most 96 registers; past that (FP32 pages of
+// K > 128, 16-bit ones at Q > 4) three waves spilled, and the bound is two (K =
+// 256, 32 heads of V = 128, us with three waves / two: FP32 pages Q = 4, 128 rows
+// 152 / 103, Q = 1 99 / 90; BF16 pages Q = 8, 128 rows 100 / 94).
+constexpr int verify_min_waves(int e, int j, int qm, int tile) {
+  const int buffers = 2 * verify_block_rows(e, j, qm) / 4 * j * 4, operands = (2 * qm + 3) / 4 * j * e;
+  return tile < 128 ? 1 : buffers + operands <= 96 ? 3 : 2;
+}
 template <typename S, typename A, int J, int QM, bool DEFER, int TILE>
-__global__ __launch_bounds__(kVerifyThreads, TILE == 128 ? 3 : 1) void verify_kernel(VerifyArgs a) {
+__global__ __launch_bounds__(kVerifyThreads, verify_min_waves(Chunk<S>::E, J, QM, TILE)) void verify_kernel(VerifyArgs a) {
   __shared__ VerifyLds<QM, 16 * Chunk<S>::E * J, DEFER, TILE> lds;
   warm_kernel_args<int(sizeof(VerifyArgs))>();
   if (DEFER || int(blockIdx.y) < a.nt_rows)  // the deferred verify: every row (see verify.hip)

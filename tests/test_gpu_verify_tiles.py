@@ -37,6 +37,14 @@ def test_batches_around_each_line(dev, B, HV, V, Q):
     _run_and_check(_problem(B, 4, HV, 128, V, Q, seed=B + V, null_rows=(1,)), dev)
 
 
+@pytest.mark.parametrize("B,K,Q,state", [(65, 256, 1, torch.float32), (41, 136, 2, torch.float32),
+                                         (41, 256, 4, torch.float32), (17, 256, 8, torch.float32),
+                                         (17, 160, 6, torch.bfloat16)])
+def test_long_tiles_of_wide_rows(dev, B, K, Q, state):
+    # 128-row tiles with K > 128: two waves per SIMD, and 8-row blocks at Q = 8 (verify_block_rows).
+    _run_and_check(_problem(B, 4, 32, K, 120, Q, seed=B + K, state_dtype=state), dev)
+
+
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Q,state", [(1, torch.float32), (2, torch.bfloat16), (4, torch.float32), (4, torch.bfloat16),
                                      (8, torch.float32)])
