@@ -227,8 +227,7 @@ static int verify_impl(const void *q, const void *k, const void *v, const void *
     a.softplus_beta = gating->softplus_beta;
     a.softplus_threshold = gating->softplus_threshold;
   }
-  int j = 1;
-  while (16 * E * j < K) j *= 2;
+  const int kp = K <= 64 ? 64 : K <= 128 ? 128 : 256;
   const int qm = Q <= 1 ? 1 : Q <= 2 ? 2 : Q <= 4 ? 4 : 8;
   const int tile = verify_tile(rows, value_heads, V, qm, pending != nullptr);
   a.NVT = int32_t((V + tile - 1) / tile);
@@ -255,9 +254,9 @@ static int verify_impl(const void *q, const void *k, const void *v, const void *
   auto s = static_cast<hipStream_t>(stream);
   const dim3 gd(static_cast<unsigned>(a.NVT * value_heads), static_cast<unsigned>(rows), 1u);
   switch (ext->state_dtype) {
-    case GDN_DT_BF16: launch_verify_state<bf16>(act, j, tile, qm, pending != nullptr, gd, s, a); break;
-    case GDN_DT_F16: launch_verify_state<f16>(act, j, tile, qm, pending != nullptr, gd, s, a); break;
-    default: launch_verify_state<float>(act, j, tile, qm, pending != nullptr, gd, s, a); break;
+    case GDN_DT_BF16: launch_verify_state<bf16>(act, kp, tile, qm, pending != nullptr, gd, s, a); break;
+    case GDN_DT_F16: launch_verify_state<f16>(act, kp, tile, qm, pending != nullptr, gd, s, a); break;
+    default: launch_verify_state<float>(act, kp, tile, qm, pending != nullptr, gd, s, a); break;
   }
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) {

@@ -27,7 +27,7 @@
 // 4-row by 4-column outer product: lane l = 4*kb + i holds row i of A and
 // column i of B of block kb, and register r of D holds (row r, column i).
 // Here block kb takes the 16-byte chunks 16j + kb of four state rows (A) and of
-// four of the vectors k, q~ (B), so
+// four of the vectors k, q~ (B) (16-bit pages of K <= 64: see RowLanes), so
 //   * a load gives the 64 lanes four whole runs of 256 bytes, one per state
 //     row, straight in the operand layout (the 16x16x4 instruction's layout is
 //     16 rows x 64 bytes per load: half of 16 lines, which is why that form
@@ -42,8 +42,8 @@
 // (reduce_rows: 3 lane swaps, 3 adds and 2 rotated adds per 4x4 tile).
 //
 // Template parameters: S state element type, A activation type (q, k, v and
-// the key record / output when they share it), J 16-byte chunks per lane per
-// row (K <= 16*E*J), QM window capacity (Q <= QM).
+// the key record / output when they share it), KP the padded K (64, 128 or 256),
+// QM window capacity (Q <= QM).
 #pragma once
 
 #include "gdn_common.cuh"
@@ -249,8 +249,26 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The sum over the 16 blocks kb = lane / 4 of a value per (block, lane % 4),
-// in every lane.
+// Lanes of a state row: all 16 blocks share one, except that a row of up to 64
+// 16-bit elements (128 bytes) is split over 8 of them and an instruction's two
+// halves take two sets of four rows. A load is then eight runs of 128 bytes, one
+// line each, and a result is summed over 8 blocks; over 16 blocks half of the
+// lanes and of the products were padding. K = 64, 32 heads, one layer, us over 16 /
+// 8 blocks, 64-row tiles: FP16 V = 64, Q = 4, 256 rows 35.8 / 26.4; V = 192, Q = 8,
+// 256 rows 163 / 105; deferred, V = 192, Q = 4, 256 rows 159 / 100.
+// FP32 rows of K = 64 fill 16 blocks, and are left there: over 8 a lane holds
+// twice the operands, and small launches and Q = 8 got slower (4 rows Q = 1 3.7 /
+// 4.1, V = 128 256 rows Q = 8 82 / 89).
+template <typename S, int KP>
+struct RowLanes {
+  static constexpr int E = Chunk<S>::E;       // elements per 16-byte chunk
+  static constexpr int N = sizeof(S) == 2 && KP == 64 ? 8 : 16;  // blocks of a row
+  static constexpr int J = KP / (N * E);      // chunks per lane per row
+  static constexpr int ROWS = 64 / N;         // rows of a load
+};
+
+// The sum over a row's N blocks (16: all of kb = lane / 4, 8: kb % 8) of a value
+// per (block, lane % 4), in every lane of the row.
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float x) {
   return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
@@ -264,16 +282,22 @@ __device__ __forceinline__ float swap_add16(float x, float y) {  // even 16-lane
   const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
   return __uint_as_float(p[0]) + __uint_as_float(p[1]);
 }
+template <int N>
 __device__ __forceinline__ float sum_blocks(float x) {
-  x = swap_add32(x, x);
+  if constexpr (N == 16) x = swap_add32(x, x);
   x = swap_add16(x, x);
   return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
 }
-// The same for the four registers of a 4x4 result tile at once: lane
-// 16*r + 4*any + i gets the sum of row r, column i.
+// The same for the four registers of a 4x4 result tile at once. N = 16: lane
+// 16*r + 4*any + i gets the sum of row r, column i. N = 8: `lo` gets rows 0 (lanes
+// of even 16) and 1 (odd), `hi` rows 2 and 3, each half of the wave its own tile.
 __device__ __forceinline__ float reduce_rows(f32x4 a) {
   const float x = swap_add16(swap_add32(a[0], a[2]), swap_add32(a[1], a[3]));
   return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
+}
+__device__ __forceinline__ void reduce_rows8(f32x4 a, float &lo, float &hi) {
+  lo = dpp_add<kRowRor4>(dpp_add<kRowRor8>(swap_add16(a[0], a[1])));
+  hi = dpp_add<kRowRor4>(dpp_add<kRowRor8>(swap_add16(a[2], a[3])));
 }
 
 // DEFER: before verifying, apply the previous step's commit for this row (the
@@ -293,23 +317,26 @@ struct __align__(16) VerifyLds {
   float pc[DEFER ? QM : 1][DEFER ? HALF : 1];              // and its corrections of the tile's rows
 };
 
-// Rows of a block: 16, or 8 where the two block buffers (32J registers a lane at
+// Rows of a block: 16, or 8 where the two block buffers (128 registers a lane at
 // 16 rows) and the 64 registers of B operands of FP32 pages of K > 128 at Q > 4
 // would take a wave all its SIMD's registers: at 16 rows that kernel had one
 // wave per SIMD, or spilled (K = 256, Q = 8, 32 heads, 64 rows: 143 us held to
 // three waves, 69 to two, 65 with blocks of 8 rows).
-__host__ __device__ constexpr int verify_block_rows(int e, int j, int qm) { return e == 4 && j == 4 && qm == 8 ? 8 : 16; }
+template <typename S, int KP>
+__host__ __device__ constexpr int verify_block_rows(int qm) {
+  return sizeof(S) == 4 && KP == 256 && qm == 8 ? 8 : 16;
+}
 
-template <typename S, typename A, int J, int QM, bool DEFER, bool NT, int TILE>
-__device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 16 * Chunk<S>::E * J, DEFER, TILE> &L) {
+template <typename S, typename A, int KP, int QM, bool DEFER, bool NT, int TILE>
+__device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, KP, DEFER, TILE> &L) {
   static_assert(!DEFER || TILE <= 64, "the pending corrections cover one half tile");
-  constexpr int E = Chunk<S>::E;       // elements per 16-byte chunk
-  constexpr int KP = 16 * E * J;       // K padded to 16 blocks x J chunks x E
+  using R = RowLanes<S, KP>;
+  constexpr int E = R::E, J = R::J;    // elements of a chunk, chunks per lane per row
   constexpr int NV = 2 * QM;           // columns: k_0 .. k_{QM-1}, q~_0 .. q~_{QM-1}
   constexpr int CG = (NV + 3) / 4;     // groups of 4 columns
   constexpr int CGK = (QM + 3) / 4;    // column groups that hold a k
-  constexpr int BROWS = verify_block_rows(E, J, QM);
-  constexpr int BG = BROWS / 4;        // 4-row groups of a block
+  constexpr int BROWS = verify_block_rows<S, KP>(QM);
+  constexpr int BG = BROWS / R::ROWS;  // loads of a block per chunk
   constexpr int NRB = TILE / BROWS;    // blocks per tile
   constexpr int HALF = TILE < 64 ? TILE : 64;  // rows of one recurrence (one per lane)
   constexpr int HRB = HALF / BROWS;
@@ -455,8 +482,9 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
   const bool verify_row = !null_slot && valid_mask != 0;
   if (!verify_row) valid_mask = 0;
 
-  const int kb = lane >> 2, ij = lane & 3;     // block; state row / column within its 4
-  const int q16 = lane >> 4, bq = kb & 3;      // after reduce_rows: state row, and the copy's number
+  // Block within its row, row / column within its 4, and the row's place in a load.
+  const int kb = (lane >> 2) & (R::N - 1), ij = lane & 3, lr = R::N == 16 ? ij : 4 * (lane >> 5) + ij;
+  const int bq = (lane >> 2) & 3;  // a result's copy (reduce_rows)
 
   // ---- 2. small loads first: the lane's chunks of k and q, v of its rows ----
   // Column c = 4*cg + ij is k_c, or q_{c - QM}.
@@ -472,7 +500,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
     const bool on = (col < NV) & (((valid_mask >> t) & 1u) != 0);
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const int kk = (16 * j + kb) * E;
+      const int kk = (R::N * j + kb) * E;
       const int off = (t * (is_q ? a.q_ts : a.k_ts) + h * K + kk) * AS;
       // With QM a multiple of 4 a group is all k or all q; else one of two
       // loads reads out of range.
@@ -531,7 +559,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
   // Buffer loads: one resource per (slot, head) tile, a 32-bit per-lane offset
   // per chunk and the block step in the scalar offset. Rows >= V lie past the
   // resource's extent and read as zero; chunks >= K get an out-of-range offset.
-  // Register g*J + j of a block: row 4g + ij, chunk 16j + kb.
+  // Register g*J + j of a block: row ROWS*g + lr, chunk N*j + kb.
   const int tile_rows = V - row0 < TILE ? V - row0 : TILE;
   const int tile_bytes = tile_rows * a.state_vs * int(sizeof(S));
   auto tile_rsrc = [&](int64_t page, bool use) {
@@ -549,10 +577,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
   // A 24-bit product (row_bytes < 2^24, checked on the host): a full multiply
   // here became a 64-bit multiply-add whose unused high addend was a register
   // with a load in flight, and waiting for it held back the first state loads.
-  const int lane_off = int(__umul24(unsigned(ij), unsigned(row_bytes))) + kb * 16;
+  const int lane_off = int(__umul24(unsigned(lr), unsigned(row_bytes))) + kb * 16;
   constexpr int BR = BG * J;  // 16-byte chunks per lane of a block
-  auto s_voff = [&](int j) { return (16 * j + kb) * E < K ? lane_off : kOutOfRange; };
-  auto s_soff = [&](int rb, int g, int j) { return (rb * BROWS + 4 * g) * row_bytes + j * 256; };
+  auto s_voff = [&](int j) { return (R::N * j + kb) * E < K ? lane_off : kOutOfRange; };
+  auto s_soff = [&](int rb, int g, int j) { return (rb * BROWS + R::ROWS * g) * row_bytes + j * R::N * 16; };
   // One form for every K, and every block is loaded (blocks past V read as
   // zero): a conditional load would leave a path on which it was not issued,
   // and the wait counts of every later MFMA would have to assume that path,
@@ -633,7 +661,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
       for (int j = 0; j < J; ++j)
 #pragma unroll
         for (int e = 0; e < E; ++e) ss = __builtin_fmaf(m[cg][j][e], m[cg][j][e], ss);
-      const float inv = rsqrtf(sum_blocks(ss) + 1e-6f);
+      const float inv = rsqrtf(sum_blocks<R::N>(ss) + 1e-6f);
 #pragma unroll
       for (int j = 0; j < J; ++j)
 #pragma unroll
@@ -646,10 +674,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
 #pragma unroll
     for (int cg = 0; cg < CGK; ++cg) {
       const int t = 4 * cg + ij;
-      if (t < QM && ((valid_mask >> (t & 31)) & 1u)) {
+      if (t < QM && ((valid_mask >> (t & 31)) & 1u) && (R::N == 16 || lane < 32)) {  // N = 8: both halves hold it
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-          const int kk = (16 * j + kb) * E;
+          const int kk = (R::N * j + kb) * E;
           if (kk < K) {
             const int64_t base = int64_t(b) * z->key_rs + int64_t(key_head) * z->key_hs + int64_t(t) * z->key_ts + kk;
 #pragma unroll
@@ -674,7 +702,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
     if (lane < QM && ((valid_mask >> lane) & 1u))
       z->decay[int64_t(b) * z->decay_rs + int64_t(hv) * z->decay_hs + int64_t(lane) * z->decay_ts] = dl;
   }
-  // k_s . column c of lane 16*(s % 4) + c % 4 of gram[s / 4][c / 4].
+  // k_s . column c in lane gram_lane(s, c) of gram[s / 4][c / 4].
+  auto gram_lane = [](int s, int c) {
+    return (R::N == 16 ? 16 * (s & 3) : 16 * (s & 1) + 4 * ((s >> 1) & 1)) + (c & 3);
+  };
   float gram[CGK][CG];
 #pragma unroll
   for (int s = 0; s < CGK; ++s)
@@ -685,10 +716,16 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
       for (int j = 0; j < J; ++j)
 #pragma unroll
         for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(m[s][j][e], m[cg][j][e], acc, 0, 0, 0);
-      gram[s][cg] = reduce_rows(acc);
+      if constexpr (R::N == 16) {
+        gram[s][cg] = reduce_rows(acc);
+      } else {
+        float lo, hi;
+        reduce_rows8(acc, lo, hi);
+        gram[s][cg] = (bq & 1) != 0 ? hi : lo;
+      }
     }
   auto dot = [&](int s, int c) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gram[s / 4][c / 4]), 16 * (s & 3) + (c & 3)));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gram[s / 4][c / 4]), gram_lane(s, c)));
   };
   // DEFER: the pending keys and corrections to LDS, the decays to scalars. A
   // lane's chunks of the keys stay in registers where they are few.
@@ -721,7 +758,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
 #pragma unroll
         for (int j = 0; j < J; ++j)
 #pragma unroll
-          for (int e = 0; e < E; ++e) pkr[t][j][e] = pk_lds[t][(16 * j + kb) * E + e];
+          for (int e = 0; e < E; ++e) pkr[t][j][e] = pk_lds[t][(R::N * j + kb) * E + e];
     }
   }
 
@@ -747,7 +784,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
             const float d = pdec[t];
             float c[BG];
 #pragma unroll
-            for (int g = 0; g < BG; ++g) c[g] = pc_lds[t][(rb & (HRB - 1)) * BROWS + 4 * g + ij];
+            for (int g = 0; g < BG; ++g) c[g] = pc_lds[t][(rb & (HRB - 1)) * BROWS + R::ROWS * g + lr];
 #pragma unroll
             for (int j = 0; j < J; ++j) {
               float kv[E];
@@ -756,7 +793,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
                 if constexpr (PK_REGS)
                   kv[e] = pkr[t][j][e];
                 else
-                  kv[e] = pk_lds[t][(16 * j + kb) * E + e];
+                  kv[e] = pk_lds[t][(R::N * j + kb) * E + e];
               }
 #pragma unroll
               for (int g = 0; g < BG; ++g)
@@ -802,17 +839,28 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
           for (int cg = 0; cg < CG; ++cg)
             acc[cg] = __builtin_amdgcn_mfma_f32_4x4x1f32(x, m[cg][j][e], acc[cg], 0, 0, 0);
         }
-      // Rows 4g .. 4g+3: every copy holds the sums; copy g keeps them.
+      // Every copy holds the sums; one keeps them: copy g those of rows 4g .. 4g+3
+      // (N = 16), copies 2g and 2g + 1 those of rows 8g + {0, 1} and 8g + {2, 3} of
+      // each half's four.
 #pragma unroll
       for (int cg = 0; cg < CG; ++cg) {
-        const float r = reduce_rows(acc[cg]);
-        y[cg] = g == 0 || bq == g ? r : y[cg];
+        if constexpr (R::N == 16) {
+          const float r = reduce_rows(acc[cg]);
+          y[cg] = g == 0 || bq == g ? r : y[cg];
+        } else {
+          float lo, hi;
+          reduce_rows8(acc[cg], lo, hi);
+          y[cg] = g == 0 || bq == 2 * g ? lo : y[cg];
+          y[cg] = bq == 2 * g + 1 ? hi : y[cg];
+        }
       }
     }
-    const int row = (rb & (HRB - 1)) * BROWS + 4 * bq + q16;
+    const int row = (rb & (HRB - 1)) * BROWS +
+                    (R::N == 16 ? 4 * bq + (lane >> 4)
+                                : 8 * (bq >> 1) + 4 * (lane >> 5) + 2 * (bq & 1) + ((lane >> 4) & 1));
 #pragma unroll
     for (int cg = 0; cg < CG; ++cg)
-      if ((BG == 4 || bq < BG) && (NV % 4 == 0 || 4 * cg + ij < NV)) d_lds[row][4 * cg + ij] = y[cg];
+      if ((BROWS == 16 || bq < BG) && (NV % 4 == 0 || 4 * cg + ij < NV)) d_lds[row][4 * cg + ij] = y[cg];
   };
   // Outputs and corrections go out through buffer stores that are issued for
   // every token and lane (an invalid one gets an out-of-range offset and is
@@ -910,87 +958,86 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, 1
 // K > 128, 16-bit ones at Q > 4) three waves spilled, and the bound is two (K =
 // 256, 32 heads of V = 128, us with three waves / two: FP32 pages Q = 4, 128 rows
 // 152 / 103, Q = 1 99 / 90; BF16 pages Q = 8, 128 rows 100 / 94).
-constexpr int verify_min_waves(int e, int j, int qm, int tile) {
-  const int buffers = 2 * verify_block_rows(e, j, qm) / 4 * j * 4, operands = (2 * qm + 3) / 4 * j * e;
+template <typename S, int KP>
+constexpr int verify_min_waves(int qm, int tile) {
+  using R = RowLanes<S, KP>;
+  const int buffers = 2 * (verify_block_rows<S, KP>(qm) / R::ROWS) * R::J * 4;
+  const int operands = (2 * qm + 3) / 4 * R::J * R::E;
   return tile < 128 ? 1 : buffers + operands <= 96 ? 3 : 2;
 }
-template <typename S, typename A, int J, int QM, bool DEFER, int TILE>
-__global__ __launch_bounds__(kVerifyThreads, verify_min_waves(Chunk<S>::E, J, QM, TILE)) void verify_kernel(VerifyArgs a) {
-  __shared__ VerifyLds<QM, 16 * Chunk<S>::E * J, DEFER, TILE> lds;
+template <typename S, typename A, int KP, int QM, bool DEFER, int TILE>
+__global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, KP>(QM, TILE))) void verify_kernel(VerifyArgs a) {
+  __shared__ VerifyLds<QM, KP, DEFER, TILE> lds;
   warm_kernel_args<int(sizeof(VerifyArgs))>();
   if (DEFER || int(blockIdx.y) < a.nt_rows)  // the deferred verify: every row (see verify.hip)
-    verify_wave<S, A, J, QM, DEFER, true, TILE>(a, lds);
+    verify_wave<S, A, KP, QM, DEFER, true, TILE>(a, lds);
   else
-    verify_wave<S, A, J, QM, DEFER, false, TILE>(a, lds);
+    verify_wave<S, A, KP, QM, DEFER, false, TILE>(a, lds);
 }
 
 // Launch for one state type; defined per state type in verify_<state>.hip.
 template <typename S>
-void launch_verify_state(int act_dt, int j, int tile, int qm, bool deferred, dim3 grid, hipStream_t s,
+void launch_verify_state(int act_dt, int kp, int tile, int qm, bool deferred, dim3 grid, hipStream_t s,
                          const VerifyArgs &a);
 
-template <typename S, typename A, int J, bool DEFER, int TILE>
+template <typename S, typename A, int KP, bool DEFER, int TILE>
 static void launch_verify_q(int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
   const dim3 wg(kVerifyThreads);
   switch (qm) {
-    case 1: hipLaunchKernelGGL((verify_kernel<S, A, J, 1, DEFER, TILE>), grid, wg, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((verify_kernel<S, A, J, 2, DEFER, TILE>), grid, wg, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((verify_kernel<S, A, J, 4, DEFER, TILE>), grid, wg, 0, s, a); break;
-    default: hipLaunchKernelGGL((verify_kernel<S, A, J, 8, DEFER, TILE>), grid, wg, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((verify_kernel<S, A, KP, 1, DEFER, TILE>), grid, wg, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((verify_kernel<S, A, KP, 2, DEFER, TILE>), grid, wg, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((verify_kernel<S, A, KP, 4, DEFER, TILE>), grid, wg, 0, s, a); break;
+    default: hipLaunchKernelGGL((verify_kernel<S, A, KP, 8, DEFER, TILE>), grid, wg, 0, s, a); break;
   }
 }
 
-template <typename S, typename A, int J, bool DEFER>
+template <typename S, typename A, int KP, bool DEFER>
 static void launch_verify_tile(int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
   switch (tile) {
-    case 16: launch_verify_q<S, A, J, DEFER, 16>(qm, grid, s, a); break;
-    case 64: launch_verify_q<S, A, J, DEFER, 64>(qm, grid, s, a); break;
-    default: launch_verify_q<S, A, J, DEFER, DEFER ? 32 : 128>(qm, grid, s, a); break;
+    case 16: launch_verify_q<S, A, KP, DEFER, 16>(qm, grid, s, a); break;
+    case 64: launch_verify_q<S, A, KP, DEFER, 64>(qm, grid, s, a); break;
+    default: launch_verify_q<S, A, KP, DEFER, DEFER ? 32 : 128>(qm, grid, s, a); break;
   }
 }
 
-// J: 16-byte chunks per lane per row, KP = 16 * E * J <= 256, so J <= 4 for
-// f32 state and J <= 2 for 16-bit state.
 template <typename S, typename A, bool DEFER>
-static void launch_verify_j(int j, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
-  switch (j) {
-    case 1: launch_verify_tile<S, A, 1, DEFER>(tile, qm, grid, s, a); break;
-    case 2: launch_verify_tile<S, A, 2, DEFER>(tile, qm, grid, s, a); break;
-    default:
-      if constexpr (Chunk<S>::E == 4) launch_verify_tile<S, A, 4, DEFER>(tile, qm, grid, s, a);
-      break;
+static void launch_verify_kp(int kp, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
+  switch (kp) {
+    case 64: launch_verify_tile<S, A, 64, DEFER>(tile, qm, grid, s, a); break;
+    case 128: launch_verify_tile<S, A, 128, DEFER>(tile, qm, grid, s, a); break;
+    default: launch_verify_tile<S, A, 256, DEFER>(tile, qm, grid, s, a); break;
   }
 }
 
 template <typename S, bool DEFER>
-static void launch_verify_act(int act_dt, int j, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
+static void launch_verify_act(int act_dt, int kp, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a) {
   switch (act_dt) {
-    case GDN_DT_BF16: launch_verify_j<S, bf16, DEFER>(j, tile, qm, grid, s, a); break;
-    case GDN_DT_F16: launch_verify_j<S, f16, DEFER>(j, tile, qm, grid, s, a); break;
-    default: launch_verify_j<S, float, DEFER>(j, tile, qm, grid, s, a); break;
+    case GDN_DT_BF16: launch_verify_kp<S, bf16, DEFER>(kp, tile, qm, grid, s, a); break;
+    case GDN_DT_F16: launch_verify_kp<S, f16, DEFER>(kp, tile, qm, grid, s, a); break;
+    default: launch_verify_kp<S, float, DEFER>(kp, tile, qm, grid, s, a); break;
   }
 }
 
 // The deferred-commit kernels of each state type live in a translation unit of
 // their own (verify_<state>_deferred.hip), so the halves compile in parallel.
 template <typename S>
-void launch_verify_deferred(int act_dt, int j, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a);
+void launch_verify_deferred(int act_dt, int kp, int tile, int qm, dim3 grid, hipStream_t s, const VerifyArgs &a);
 
 #define GDN_DEFINE_VERIFY_LAUNCH(STATE)                                                                \
   template <>                                                                                          \
-  void launch_verify_state<STATE>(int act_dt, int j, int tile, int qm, bool deferred, dim3 grid, hipStream_t s, \
+  void launch_verify_state<STATE>(int act_dt, int kp, int tile, int qm, bool deferred, dim3 grid, hipStream_t s, \
                                   const VerifyArgs &a) {                                               \
     if (deferred)                                                                                      \
-      launch_verify_deferred<STATE>(act_dt, j, tile, qm, grid, s, a);                                        \
+      launch_verify_deferred<STATE>(act_dt, kp, tile, qm, grid, s, a);                                        \
     else                                                                                               \
-      launch_verify_act<STATE, false>(act_dt, j, tile, qm, grid, s, a);                                      \
+      launch_verify_act<STATE, false>(act_dt, kp, tile, qm, grid, s, a);                                      \
   }
 
 #define GDN_DEFINE_VERIFY_DEFERRED_LAUNCH(STATE)                                                         \
   template <>                                                                                            \
-  void launch_verify_deferred<STATE>(int act_dt, int j, int tile, int qm, dim3 grid, hipStream_t s,                \
+  void launch_verify_deferred<STATE>(int act_dt, int kp, int tile, int qm, dim3 grid, hipStream_t s,                \
                                      const VerifyArgs &a) {                                              \
-    launch_verify_act<STATE, true>(act_dt, j, tile, qm, grid, s, a);                                           \
+    launch_verify_act<STATE, true>(act_dt, kp, tile, qm, grid, s, a);                                           \
   }
 
 }  // namespace gdn

@@ -45,6 +45,16 @@ def test_long_tiles_of_wide_rows(dev, B, K, Q, state):
     _run_and_check(_problem(B, 4, 32, K, 120, Q, seed=B + K, state_dtype=state), dev)
 
 
+@pytest.mark.parametrize("K", [8, 48, 64])
+@pytest.mark.parametrize("Q", [1, 2, 4, 8])
+@pytest.mark.parametrize("state,act", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                       (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("B,V", [(3, 33), (14, 120), (66, 120)])
+def test_narrow_16bit_rows(dev, K, Q, state, act, B, V):
+    # Pages of K <= 64 16-bit elements: a row over 8 blocks, tiles of 16, 64 and 128.
+    _run_and_check(_problem(B, 2, 32, K, V, Q, seed=B + K + Q, state_dtype=state, act=act), dev)
+
+
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Q,state", [(1, torch.float32), (2, torch.bfloat16), (4, torch.float32), (4, torch.bfloat16),
                                      (8, torch.float32)])

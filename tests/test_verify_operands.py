@@ -1,6 +1,6 @@
 """The verify kernel's lane arithmetic (csrc/verify_kernel.cuh), restated on the
-CPU: `reduce_rows` over the 16 blocks of a 4x4x1 matrix instruction, the loads'
-cover of a 16-row block, `udiv`, and the runs of 16-bit elements that start in
+CPU: `reduce_rows` over the 16 (or 8) blocks of a 4x4x1 matrix instruction, the
+loads' cover of a block of rows, `udiv`, and the runs of 16-bit elements that start in
 either half of a dword (`load_run`)."""
 
 import random
@@ -37,17 +37,63 @@ def test_reduce_rows_sums_the_blocks():
         assert x[lane] == sum(acc[r][4 * kb + col] for kb in range(16))
 
 
-@pytest.mark.parametrize("J", [1, 2, 4])
-def test_block_loads_are_whole_row_runs(J):
-    """Register g*J + j of lane 4*kb + ij holds chunk 16j + kb of row 4g + ij: each
-    chunk once, every load four runs of 16 consecutive chunks."""
+def test_reduce_rows8_sums_the_blocks_of_each_half():
+    """Rows over 8 blocks: lo holds rows 0 (even 16 lanes) and 1 (odd) of each half's
+    tile, hi rows 2 and 3."""
+    rng = random.Random(3)
+    acc = [[rng.randrange(1 << 20) for _ in range(64)] for _ in range(4)]
+    for first in (0, 2):
+        x = _add(_swap16(acc[first], acc[first + 1]))
+        x = _add((x, _ror(x, 8)))
+        x = _add((x, _ror(x, 4)))
+        for lane in range(64):
+            half, r, col = lane >> 5, first + ((lane >> 4) & 1), lane & 3
+            assert x[lane] == sum(acc[r][32 * half + 4 * kb + col] for kb in range(8))
+
+
+def test_result_rows_over_8_blocks():
+    """Copies 2g and 2g + 1 keep lo and hi of load g: lane and register give row
+    8*(bq >> 1) + 4*(lane >> 5) + 2*(bq & 1) + (lane >> 4 & 1), every row once per column."""
+    got = {}
+    for lane in range(64):
+        bq = (lane >> 2) & 3
+        g, hi, half = bq >> 1, bq & 1, lane >> 5
+        source = 8 * g + 4 * half + 2 * hi + ((lane >> 4) & 1)  # load g's rows 8g + 4*half + (0..3)
+        row = 8 * (bq >> 1) + 4 * (lane >> 5) + 2 * (bq & 1) + ((lane >> 4) & 1)
+        assert row == source and (row, lane & 3) not in got
+        got[row, lane & 3] = lane
+    assert len(got) == 64
+
+
+@pytest.mark.parametrize("N", [16, 8])
+def test_gram_lanes(N):
+    """gram_lane(s, c) names a lane that holds row s % 4, column c % 4 of the result."""
+    for s in range(8):
+        for c in range(16):
+            lane = (16 * (s & 3) if N == 16 else 16 * (s & 1) + 4 * ((s >> 1) & 1)) + (c & 3)
+            row = lane >> 4 if N == 16 else ((lane >> 4) & 1) + 2 * ((lane >> 2) & 1)
+            assert row == s % 4 and (lane & 3) == c % 4
+
+
+@pytest.mark.parametrize("N,J", [(16, 1), (16, 2), (16, 4), (8, 1)])
+@pytest.mark.parametrize("block", [16, 8])
+def test_block_loads_are_whole_row_runs(N, J, block):
+    """Register g*J + j of a lane holds chunk N*j + kb of row ROWS*g + lr: each chunk
+    once, every load 64 / N runs of N consecutive chunks."""
+    rows = 64 // N
+    if block % rows:
+        pytest.skip("not a block of this split")
     seen = []
-    for g in range(4):
+    for g in range(block // rows):
         for j in range(J):
-            at = [(4 * g + (lane & 3), 16 * j + (lane >> 2)) for lane in range(64)]
-            assert sorted(at) == [(4 * g + r, 16 * j + c) for r in range(4) for c in range(16)]
+            at = []
+            for lane in range(64):
+                kb, ij = (lane >> 2) & (N - 1), lane & 3
+                lr = ij if N == 16 else 4 * (lane >> 5) + ij
+                at.append((rows * g + lr, N * j + kb))
+            assert sorted(at) == [(rows * g + r, N * j + c) for r in range(rows) for c in range(N)]
             seen += at
-    assert sorted(seen) == [(r, c) for r in range(16) for c in range(16 * J)]
+    assert sorted(seen) == [(r, c) for r in range(block) for c in range(N * J)]
 
 
 def test_udiv_is_exact():
