@@ -36,7 +36,7 @@
 //     were re-read from LDS for each), loaded by each lane from q and k: no
 //     LDS staging and no barrier before the first product;
 //   * 4 columns are computed, not 16, of which Q = 4 uses 8: half the
-//     matrix-core time at Q <= 4, the same at Q = 8;
+//     matrix-core time at Q <= 4, the same at Q = 8 (see verify_wide);
 //   * the Gram matrix is the same instruction on the B registers themselves.
 // The 16 blocks' partial sums are added across lanes at the end of four rows
 // (reduce_rows: 3 lane swaps, 3 adds and 2 rotated adds per 4x4 tile).
@@ -288,7 +288,11 @@ __device__ __forceinline__ float sum_blocks(float x) {
   x = swap_add16(x, x);
   return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
 }
-// The same for the four registers of a 4x4 result tile at once. N = 16: lane
+__device__ __forceinline__ float sum_quarters(float x) {  // over the lanes of equal l % 16
+  x = swap_add32(x, x);
+  return swap_add16(x, x);
+}
+// The sum for the four registers of a 4x4 result tile at once. N = 16: lane
 // 16*r + 4*any + i gets the sum of row r, column i. N = 8: `lo` gets rows 0 (lanes
 // of even 16) and 1 (odd), `hi` rows 2 and 3, each half of the wave its own tile.
 __device__ __forceinline__ float reduce_rows(f32x4 a) {
@@ -309,9 +313,10 @@ __device__ __forceinline__ void reduce_rows8(f32x4 a, float &lo, float &hi) {
 // the stored page is. Each state page is read once per step instead of twice.
 // The wave's LDS, declared once per kernel and shared by both cache-policy
 // bodies below (a __shared__ array inside each would be allocated twice).
-template <int QM, int KP, bool DEFER, int TILE>
+template <int QM, int KP, bool DEFER, int TILE, int STAGE>
 struct __align__(16) VerifyLds {
   static constexpr int HALF = TILE < 64 ? TILE : 64;
+  uint4 stage[STAGE];         // one block of rows on its way to the 16x16x4 layout
   float d[HALF][2 * QM + 1];  // GEMV results of one half tile
   __align__(16) float pk[DEFER ? QM : 1][DEFER ? KP : 1];  // pending commit's keys
   float pc[DEFER ? QM : 1][DEFER ? HALF : 1];              // and its corrections of the tile's rows
@@ -327,14 +332,40 @@ __host__ __device__ constexpr int verify_block_rows(int qm) {
   return sizeof(S) == 4 && KP == 256 && qm == 8 ? 8 : 16;
 }
 
+// Windows of more than four tokens have 16 columns, a whole 16x16x4 instruction:
+// the same matrix-core time as 4x4x1 ones and no cross-lane sums, which are ten
+// instructions per four rows and four columns. Tiles of 64 rows and up whose rows
+// are at most 256 bytes are bound by instructions there, so their blocks go
+// through LDS into that layout (lane l holds row l % 16, chunks 4j + l / 16): one
+// write and one read per load of 1 KiB. One layer of 32 heads, Q = 8, us with 4x4x1
+// / 16x16x4: FP16 K = 128, V = 128, 64 rows 34.4 / 28.4, 256 rows 108 / 89; FP16 K = 64,
+// V = 192, 256 rows 103 / 82; BF16 K = 64, V = 128, 256 rows 68 / 58; FP32 K = 64, V =
+// 128, 32 rows 18.8 / 16.0, 256 rows 81 / 75. Tiles of 16 rows are a chain of
+// latencies that the detour lengthens (BF16 K = 128, 4 rows 7.4 / 9.0), and the
+// deferred verify is bound by its fold (BF16 K = 128, 64 rows 54.6 / 58.0).
+template <typename S, int KP>
+__host__ __device__ constexpr bool verify_wide(int qm, bool defer, int tile) {
+  return qm == 8 && !defer && tile >= 64 && KP * int(sizeof(S)) <= 256;
+}
+template <typename S, int KP>
+__host__ __device__ constexpr int verify_stage(int qm, bool defer, int tile) {  // chunks of a staged block
+  return verify_wide<S, KP>(qm, defer, tile) ? 16 * KP / Chunk<S>::E : 1;
+}
+
 template <typename S, typename A, int KP, int QM, bool DEFER, bool NT, int TILE>
-__device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, KP, DEFER, TILE> &L) {
+__device__ __forceinline__ void verify_wave(const VerifyArgs &a,
+                                            VerifyLds<QM, KP, DEFER, TILE, verify_stage<S, KP>(QM, DEFER, TILE)> &L) {
   static_assert(!DEFER || TILE <= 64, "the pending corrections cover one half tile");
   using R = RowLanes<S, KP>;
   constexpr int E = R::E, J = R::J;    // elements of a chunk, chunks per lane per row
   constexpr int NV = 2 * QM;           // columns: k_0 .. k_{QM-1}, q~_0 .. q~_{QM-1}
-  constexpr int CG = (NV + 3) / 4;     // groups of 4 columns
-  constexpr int CGK = (QM + 3) / 4;    // column groups that hold a k
+  constexpr bool WIDE = verify_wide<S, KP>(QM, DEFER, TILE);
+  constexpr int CW = WIDE ? 16 : 4;            // columns of a group: one instruction's
+  constexpr int CG = (NV + CW - 1) / CW;       // groups of columns
+  constexpr int CGK = (QM + CW - 1) / CW;      // column groups that hold a k
+  constexpr int CN = WIDE ? 4 : R::N;          // lanes that share a column's vector
+  constexpr int CJ = KP / (CN * E);            // chunks of it per lane
+  constexpr bool MIXED = QM % CW != 0;         // a group may hold k and q columns
   constexpr int BROWS = verify_block_rows<S, KP>(QM);
   constexpr int BG = BROWS / R::ROWS;  // loads of a block per chunk
   constexpr int NRB = TILE / BROWS;    // blocks per tile
@@ -485,27 +516,27 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
   // Block within its row, row / column within its 4, and the row's place in a load.
   const int kb = (lane >> 2) & (R::N - 1), ij = lane & 3, lr = R::N == 16 ? ij : 4 * (lane >> 5) + ij;
   const int bq = (lane >> 2) & 3;  // a result's copy (reduce_rows)
+  const int cl = WIDE ? lane & 15 : ij, cs = WIDE ? lane >> 4 : kb;  // column in its group, first chunk of its vector
 
   // ---- 2. small loads first: the lane's chunks of k and q, v of its rows ----
-  // Column c = 4*cg + ij is k_c, or q_{c - QM}.
+  // Column c = CW*cg + cl is k_c, or q_{c - QM}.
   const WordRsrc rq = make_word_rsrc(a.q, bos * a.q_ts * AS), rk = make_word_rsrc(a.k, bos * a.k_ts * AS);
-  RawRun<A, E> raw_q[CG][J], raw_k[CG][J];
+  RawRun<A, E> raw_q[CG][CJ], raw_k[CG][CJ];
 #pragma unroll
   for (int cg = 0; cg < CG; ++cg) {
-    const int col = 4 * cg + ij;
+    const int col = CW * cg + cl;
     const bool is_q = col >= QM;
     const int t = (is_q ? col - QM : col) & 31;
     // Non-short-circuit tests: a short-circuit chain became a branch per load,
     // with kernel arguments reloaded inside it.
     const bool on = (col < NV) & (((valid_mask >> t) & 1u) != 0);
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int kk = (R::N * j + kb) * E;
+    for (int j = 0; j < CJ; ++j) {
+      const int kk = (CN * j + cs) * E;
       const int off = (t * (is_q ? a.q_ts : a.k_ts) + h * K + kk) * AS;
-      // With QM a multiple of 4 a group is all k or all q; else one of two
-      // loads reads out of range.
-      if (QM % 4 != 0 || 4 * cg < QM) load_run<A, E>(rk, off, on & !is_q & (kk < K), raw_k[cg][j]);
-      if (QM % 4 != 0 || 4 * cg >= QM) load_run<A, E>(rq, off, on & is_q & (kk < K), raw_q[cg][j]);
+      // A group is all k or all q, or one of two loads reads out of range.
+      if (MIXED || CW * cg < QM) load_run<A, E>(rk, off, on & !is_q & (kk < K), raw_k[cg][j]);
+      if (MIXED || CW * cg >= QM) load_run<A, E>(rq, off, on & is_q & (kk < K), raw_q[cg][j]);
     }
   }
   // DEFER: the pending commit's keys (token t, 4 elements from kk) for LDS, FP32
@@ -634,22 +665,22 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
   // ---- 4. operands, records, Gram matrix ----
   const bool rec_ok = b < z->record_rows;
   const bool key_writer = rec_ok && vt == 0 && (z->key_per_value_head || hv == h * ratio);
-  float m[CG][J][E];  // the lane's chunks of its columns' vectors (B operands)
+  float m[CG][CJ][E];  // the lane's chunks of its columns' vectors (B operands)
 #pragma unroll
   for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      if constexpr (QM % 4 != 0) {
+    for (int j = 0; j < CJ; ++j) {
+      if constexpr (MIXED) {
         // One of the two was read out of range, as zeros. Their words are ORed:
         // a sum would lose the sign of a zero, and the key record holds the
         // key's own bits.
         RawRun<A, E> x = raw_k[cg][j];
 #pragma unroll
         for (int i = 0; i < int(sizeof(x.w) / 4); ++i) x.w[i] |= raw_q[cg][j].w[i];
-        if constexpr (sizeof(A) == 2) x.sh = 4 * cg + ij >= QM ? raw_q[cg][j].sh : x.sh;
+        if constexpr (sizeof(A) == 2) x.sh = CW * cg + cl >= QM ? raw_q[cg][j].sh : x.sh;
         unpack_run<A, E>(x, m[cg][j]);
       } else {
-        unpack_run<A, E>(4 * cg < QM ? raw_k[cg][j] : raw_q[cg][j], m[cg][j]);
+        unpack_run<A, E>(CW * cg < QM ? raw_k[cg][j] : raw_q[cg][j], m[cg][j]);
       }
     }
   if (z->l2norm) {
@@ -658,12 +689,12 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
     for (int cg = 0; cg < CG; ++cg) {
       float ss = 0.0f;
 #pragma unroll
-      for (int j = 0; j < J; ++j)
+      for (int j = 0; j < CJ; ++j)
 #pragma unroll
         for (int e = 0; e < E; ++e) ss = __builtin_fmaf(m[cg][j][e], m[cg][j][e], ss);
-      const float inv = rsqrtf(sum_blocks<R::N>(ss) + 1e-6f);
+      const float inv = rsqrtf((WIDE ? sum_quarters(ss) : sum_blocks<R::N>(ss)) + 1e-6f);
 #pragma unroll
-      for (int j = 0; j < J; ++j)
+      for (int j = 0; j < CJ; ++j)
 #pragma unroll
         for (int e = 0; e < E; ++e) m[cg][j][e] *= inv;
     }
@@ -673,11 +704,11 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
     const bool key_f32 = z->key_f32 != 0;
 #pragma unroll
     for (int cg = 0; cg < CGK; ++cg) {
-      const int t = 4 * cg + ij;
-      if (t < QM && ((valid_mask >> (t & 31)) & 1u) && (R::N == 16 || lane < 32)) {  // N = 8: both halves hold it
+      const int t = CW * cg + cl;
+      if (t < QM && ((valid_mask >> (t & 31)) & 1u) && (WIDE || R::N == 16 || lane < 32)) {  // N = 8: both halves hold it
 #pragma unroll
-        for (int j = 0; j < J; ++j) {
-          const int kk = (R::N * j + kb) * E;
+        for (int j = 0; j < CJ; ++j) {
+          const int kk = (CN * j + cs) * E;
           if (kk < K) {
             const int64_t base = int64_t(b) * z->key_rs + int64_t(key_head) * z->key_hs + int64_t(t) * z->key_ts + kk;
 #pragma unroll
@@ -688,10 +719,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
     }
   }
 #pragma unroll
-  for (int cg = QM / 4; cg < CG; ++cg) {
-    const float sc = 4 * cg + ij >= QM ? z->scale : 1.0f;
+  for (int cg = QM / CW; cg < CG; ++cg) {
+    const float sc = CW * cg + cl >= QM ? z->scale : 1.0f;
 #pragma unroll
-    for (int j = 0; j < J; ++j)
+    for (int j = 0; j < CJ; ++j)
 #pragma unroll
       for (int e = 0; e < E; ++e) m[cg][j][e] *= sc;
   }
@@ -702,30 +733,45 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
     if (lane < QM && ((valid_mask >> lane) & 1u))
       z->decay[int64_t(b) * z->decay_rs + int64_t(hv) * z->decay_hs + int64_t(lane) * z->decay_ts] = dl;
   }
-  // k_s . column c in lane gram_lane(s, c) of gram[s / 4][c / 4].
+  // k_s . column c in lane gram_lane(s, c) of gram[s / 4][c / 4]; WIDE: of
+  // wide_gram[s % 4] (lane l, register r: row 4*(l / 16) + r, column l % 16).
   auto gram_lane = [](int s, int c) {
-    return (R::N == 16 ? 16 * (s & 3) : 16 * (s & 1) + 4 * ((s >> 1) & 1)) + (c & 3);
+    return WIDE ? 16 * (s >> 2) + c : (R::N == 16 ? 16 * (s & 3) : 16 * (s & 1) + 4 * ((s >> 1) & 1)) + (c & 3);
   };
-  float gram[CGK][CG];
+  float gram[WIDE ? 1 : CGK][WIDE ? 1 : CG];
+  f32x4 wide_gram = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (WIDE) {
+    f32x4 odd = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int s = 0; s < CGK; ++s)
+    for (int j = 0; j < CJ; ++j)
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg) {
-      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int j = 0; j < J; ++j)
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(m[s][j][e], m[cg][j][e], acc, 0, 0, 0);
-      if constexpr (R::N == 16) {
-        gram[s][cg] = reduce_rows(acc);
-      } else {
-        float lo, hi;
-        reduce_rows8(acc, lo, hi);
-        gram[s][cg] = (bq & 1) != 0 ? hi : lo;
+      for (int e = 0; e < E; e += 2) {
+        wide_gram = __builtin_amdgcn_mfma_f32_16x16x4f32(m[0][j][e], m[0][j][e], wide_gram, 0, 0, 0);
+        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(m[0][j][e + 1], m[0][j][e + 1], odd, 0, 0, 0);
       }
-    }
+    wide_gram += odd;
+  } else {
+#pragma unroll
+    for (int s = 0; s < CGK; ++s)
+#pragma unroll
+      for (int cg = 0; cg < CG; ++cg) {
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+          for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(m[s][j][e], m[cg][j][e], acc, 0, 0, 0);
+        if constexpr (R::N == 16) {
+          gram[s][cg] = reduce_rows(acc);
+        } else {
+          float lo, hi;
+          reduce_rows8(acc, lo, hi);
+          gram[s][cg] = (bq & 1) != 0 ? hi : lo;
+        }
+      }
+  }
   auto dot = [&](int s, int c) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gram[s / 4][c / 4]), gram_lane(s, c)));
+    const float x = WIDE ? wide_gram[s & 3] : gram[WIDE ? 0 : s / 4][WIDE ? 0 : c / 4];
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), gram_lane(s, c)));
   };
   // DEFER: the pending keys and corrections to LDS, the decays to scalars. A
   // lane's chunks of the keys stay in registers where they are few.
@@ -823,6 +869,37 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
   };
 
   // ---- 5. pipelined S_0 . [k, q~] on the matrix cores, recurrence per half ----
+  // WIDE: a block's chunk c of row r sits at r*CPR + (c ^ swz(r)) of the stage: 16
+  // consecutive lanes of a write, and the 16 rows a read takes of one chunk, are
+  // in 16 different places modulo 256 bytes.
+  constexpr int CPR = KP / E;
+  auto stage_slot = [](int row, int c) {
+    return row * CPR + (c ^ (CPR == 16 ? ((row & 3) << 2) | (row >> 2) : ((row & 2) << 1) | (row >> 2)));
+  };
+  auto stage_block = [&](const uint4 (&src)[BR]) {
+    static_assert(!WIDE || (BROWS == 16 && J == 1 && (CPR == 16 || CPR == 8)), "stage_slot's rows");
+    wave_lds_sync();  // the block before has been read
+#pragma unroll
+    for (int g = 0; g < BG; ++g) L.stage[stage_slot(R::ROWS * g + lr, kb)] = src[g];
+    wave_lds_sync();
+  };
+  auto wide_block = [&](int rb) {
+    uint4 op[CJ];
+#pragma unroll
+    for (int j = 0; j < CJ; ++j) op[j] = L.stage[stage_slot(cl, 4 * j + cs)];
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, odd = acc;
+#pragma unroll
+    for (int j = 0; j < CJ; ++j)
+#pragma unroll
+      for (int e = 0; e < E; e += 2) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(chunk_elem<S>(op[j], e), m[0][j][e], acc, 0, 0, 0);
+        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(chunk_elem<S>(op[j], e + 1), m[0][j][e + 1], odd, 0, 0, 0);
+      }
+    acc += odd;
+    const int row = (rb & (HRB - 1)) * BROWS + 4 * cs;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d_lds[row + i][cl] = acc[i];
+  };
   auto gemv_block = [&](int rb, const uint4 (&src)[BR]) {
     float y[CG];
 #pragma unroll
@@ -915,13 +992,22 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a, VerifyLds<QM, K
   };
 #pragma unroll
   for (int rb = 0; rb < NRB; rb += 2) {
+    // A staged block's registers are free before its products.
     fold_block(rb, bufA);
-    gemv_block(rb, bufA);
+    if constexpr (WIDE)
+      stage_block(bufA);
+    else
+      gemv_block(rb, bufA);
     if (rb + 2 < NRB) load_block(rb + 2, bufA);
+    if constexpr (WIDE) wide_block(rb);
     if constexpr (NRB > 1) {
       fold_block(rb + 1, bufB);
-      gemv_block(rb + 1, bufB);
+      if constexpr (WIDE)
+        stage_block(bufB);
+      else
+        gemv_block(rb + 1, bufB);
       if (rb + 3 < NRB) load_block(rb + 3, bufB);
+      if constexpr (WIDE) wide_block(rb + 1);
     }
     if (TILE == 128 && rb + 2 == NRB / 2) load_v(1);  // smaller tiles have no second half
     // Every half runs its recurrence, also one past V (its rows store nothing):
@@ -967,7 +1053,7 @@ constexpr int verify_min_waves(int qm, int tile) {
 }
 template <typename S, typename A, int KP, int QM, bool DEFER, int TILE>
 __global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, KP>(QM, TILE))) void verify_kernel(VerifyArgs a) {
-  __shared__ VerifyLds<QM, KP, DEFER, TILE> lds;
+  __shared__ VerifyLds<QM, KP, DEFER, TILE, verify_stage<S, KP>(QM, DEFER, TILE)> lds;
   warm_kernel_args<int(sizeof(VerifyArgs))>();
   if (DEFER || int(blockIdx.y) < a.nt_rows)  // the deferred verify: every row (see verify.hip)
     verify_wave<S, A, KP, QM, DEFER, true, TILE>(a, lds);

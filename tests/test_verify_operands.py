@@ -131,3 +131,29 @@ def test_runs_of_16_bit_elements(N, first):
         u = (((got[i + 1] << 32) | got[i]) >> sh) & 0xFFFFFFFF
         out += [u & 0xFFFF, u >> 16]
     assert out == elems[first:first + N]
+
+
+@pytest.mark.parametrize("cpr,N,rows", [(16, 16, 4), (8, 8, 8)])
+def test_stage_slots(cpr, N, rows):
+    """The staged block of the 16x16x4 form: one slot per chunk; the 16 lanes of a
+    quarter of a write, and the 16 rows a read takes of one chunk, in 16 places
+    modulo 256 bytes; a read gives lane l row l % 16, chunk 4j + l / 16."""
+    def slot(row, c):
+        return row * cpr + (c ^ (((row & 3) << 2) | (row >> 2) if cpr == 16 else ((row & 2) << 1) | (row >> 2)))
+
+    stage = {}
+    for g in range(16 // rows):
+        at = []
+        for lane in range(64):
+            kb, ij = (lane >> 2) & (N - 1), lane & 3
+            row = rows * g + (ij if N == 16 else 4 * (lane >> 5) + ij)
+            at.append(slot(row, kb))
+            assert at[-1] not in stage
+            stage[at[-1]] = (row, kb)
+        assert all(len({x % 16 for x in at[q:q + 16]}) == 16 for q in range(0, 64, 16))
+    assert sorted(stage) == list(range(16 * cpr))
+    for j in range(cpr // 4):
+        for s in range(4):
+            at = [slot(row, 4 * j + s) for row in range(16)]
+            assert [stage[x] for x in at] == [(row, 4 * j + s) for row in range(16)]
+            assert len({x % 16 for x in at}) == 16
