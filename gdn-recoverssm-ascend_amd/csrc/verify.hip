@@ -8,29 +8,58 @@ namespace gdn {
 static bool float_dt_ok(int32_t dt) { return dt == GDN_DT_F32 || dt == GDN_DT_BF16 || dt == GDN_DT_F16; }
 
 // Rows of V per wave. A wave's life is a chain of about four memory round trips
-// (metadata, q/k, then its tile two 16-row blocks at a time), 4 us with one
-// block and 9 us with eight, so a launch that leaves the chip's 1024 SIMDs idle
-// takes short tiles; a wave's own reads of q, k, gates and its Gram matrix
-// repeat per tile, so a launch bound by memory takes long ones. Times in us of
-// one layer of several with K = V = 128 FP32 pages, Q = 4, HV = 32, tiles of 16 /
-// 64 / 128 rows: 1 row 5.4 / 7.5 / 11.2, 4 rows 5.9 / 7.6 / 11.2, 8 rows 9.1 /
-// 8.6 / 12.0, 16 rows 13.8 / 12.5 / 13.9; 64 / 128 rows: 24 rows 17.0 / 17.9, 40
-// rows (2560 waves of 64) 24.1 / 24.3, 48 rows 28.3 / 27.1, gated 37 rows 24.2 /
-// 25.2, BF16 pages 32 rows 14.7 / 15.6, 48 rows 20.8 / 20.2. At Q = 8 a wave's own
-// reads and Gram matrix are four times as large: 16 rows 16.5 / 19.9, 24 rows
-// 24.2 / 22.1. At Q = 1 they are a fraction, and 16-row tiles stay ahead up to
-// 64 rows (16 / 64 / 128: 16 rows 10.2 / 11.8 / 11.2, 64 rows 28.1 / 31.7 / 31.2,
-// 128 rows 51 / 53 / 52).
+// (metadata, q/k, then its tile two blocks at a time), 4 us with one block and 9 us
+// with eight, so a launch that leaves the chip's 1024 SIMDs idle takes short
+// tiles; a wave's own reads of q, k, gates and its Gram matrix repeat per tile, so a
+// launch bound by memory takes long ones. Times in us of one layer of several,
+// V = 128, HV = 32, FP32 pages of K = 128 unless named; the lines are in waves, so
+// that V and HV off these figures move with them (HV = 12, V = 96 and HV = 32, V = 64
+// and 192 were measured too).
 //
-// The deferred verify also writes the tile back, and a launch's time steps with
-// its rounds of resident waves (3 per SIMD, 3072): the smallest tile whose
-// waves fit one round, else 32 rows (tiles of 16 / 32 / 64 rows: 1 row 6.8 /
-// 8.4 / 10.9, 8 rows 12.1 / 13.2 / 14.2, 16 rows 18.6 / 18.1 / 18.4, 32 rows
-// 35 / 32.6 / 30.6, 64 rows 60 / 58 / 61, 128 rows 110 / 105 / 105).
-static int verify_tile(int64_t rows, int64_t value_heads, int64_t V, int qm, bool deferred) {
+// Ordinary verify, tiles of 16 / 64 / 128 rows:
+//   * 16 rows up to 1536 waves (Q > 4: 1280), one and a half a SIMD. Q = 4: 4 rows
+//     6.0 / 7.4 / 10.7, 8 rows 9.4 / 7.8 / 11.0; BF16 4 rows 5.4 / 7.4 / 10.7, 8 rows 7.7
+//     / 7.7 / 10.8; K = 64, V = 192, 4 rows (1536) 5.8 / 6.8 / 8.7; Q = 8: 4 rows 8.6 / 11.6
+//     / 17.1, 8 rows 13.0 / 12.0 / 17.4.
+//   * V <= 32: a longer tile is mostly padding (256 rows 41 / 43 / 58).
+//   * FP32 pages of K > 64 at Q = 1, where a wave's own reads are a fraction of its
+//     tile: 16 rows up to 12288 waves (24 rows 13.5 / 15.4 / 16.0, 48 rows 23.1 / 25.5 /
+//     24.1, 64 rows 27.2 / 28.3 / 26.9), K > 128 up to 4096 (16 rows 17.6 / 19.4 / 19.0,
+//     32 rows 28.5 / 26.2 / 26.0). At Q = 2 with K <= 128 they win from 4096 to 8192 waves
+//     only (8 rows 7.6 / 6.7 / 8.4, 16 rows 10.8 / 11.7 / 12.1, 32 rows 18.4 / 20.5 / 20.1,
+//     48 rows 23.6 / 25.6 / 23.1). 16-bit and K = 64 rows are shorter, and lose (BF16
+//     Q = 1, 16 rows 8.0 / 6.7 / 8.3).
+//   * 64 rows where the second half of the last 128 rows would lie past V: it takes
+//     its loads and a recurrence all the same (K = 64, 256 rows, 64 / 128: V = 64 Q = 4
+//     35 / 43, Q = 8 52 / 57; V = 192 Q = 4 79 / 92; FP16 V = 192 Q = 8 84 / 91).
+//   * else 64 rows up to 2560 waves of 64, and at Q > 4, where a wave's own work is
+//     four times as large, up to 1024. Q = 4, 64 / 128: 24 rows 17.0 / 18.1, 32 rows
+//     20.9 / 21.5, 48 rows 26.6 / 25.6; BF16 32 rows 14.9 / 15.9, 48 rows 20.5 / 20.1; Q = 8:
+//     16 rows 15.7 / 19.8, 24 rows 22.9 / 21.3; BF16 16 rows 12.5 / 16.8, 24 rows 18.7 / 18.0.
+//
+// The deferred verify also folds its tile and writes it back. Tiles of 16 / 32 / 64 rows:
+//   * 16 rows up to 3072 waves (12 rows 15.3 / 15.4 / 16.2, 16 rows 18.7 / 17.8 / 18.9;
+//     HV = 12, V = 96, 32 rows 13.1 / 14.7 / 15.3), at Q > 4, whose waves are longer, 1280
+//     (4 rows 12.2 / 14.2 / 18.3, 8 rows 17.9 / 16.1 / 20.1), and V <= 16.
+//   * 32 rows up to 3072 waves of 32, and where 64 rows would be half padding (HV = 12,
+//     V = 96, 128 rows 33.3 / 34.4 / 38.9).
+//   * 64 rows for 16-bit pages and Q > 4, bound by instructions that repeat per tile
+//     (BF16 Q = 4, 256 rows 171 / 124 / 114; Q = 8, 64 rows 92 / 78 / 68, 256 rows 335 / 273 /
+//     233); else while its waves stay within 3072 (32 rows 34.3 / 31.5 / 30.0), and 32
+//     rows past that (64 rows 60.8 / 57.6 / 60.0, 128 rows 112 / 104 / 104; 48 layers of 128
+//     rows took 5083 us at 32 rows and 5185 at 64; 256 rows 210 / 198 / 193 to 199).
+static int verify_tile(int64_t rows, int64_t value_heads, int64_t K, int64_t V, bool f32, int qm, bool deferred) {
   auto waves = [&](int tile) { return rows * value_heads * ((V + tile - 1) / tile); };
-  if (deferred) return waves(16) <= 3072 ? 16 : waves(32) <= 3072 ? 32 : waves(64) <= 3072 ? 64 : 32;
-  if (waves(16) <= (qm == 1 ? 16384 : 1280)) return 16;
+  if (deferred) {
+    if (waves(16) <= (qm == 8 ? 1280 : 3072) || V <= 16) return 16;
+    if (waves(32) <= 3072 || (V - 1) % 64 < 32) return 32;
+    return !f32 || qm == 8 || waves(64) <= 3072 ? 64 : 32;
+  }
+  const int64_t w16 = waves(16);
+  if (w16 <= (qm == 8 ? 1280 : 1536) || V <= 32) return 16;
+  if (f32 && K > 64 && qm == 1 && w16 <= (K > 128 ? 4096 : 12288)) return 16;
+  if (f32 && K > 64 && K <= 128 && qm == 2 && w16 >= 4096 && w16 <= 8192) return 16;
+  if ((V - 1) % 128 < 64) return 64;
   return waves(64) <= (qm == 8 ? 1024 : 2560) ? 64 : 128;
 }
 
@@ -229,7 +258,7 @@ static int verify_impl(const void *q, const void *k, const void *v, const void *
   }
   const int kp = K <= 64 ? 64 : K <= 128 ? 128 : 256;
   const int qm = Q <= 1 ? 1 : Q <= 2 ? 2 : Q <= 4 ? 4 : 8;
-  const int tile = verify_tile(rows, value_heads, V, qm, pending != nullptr);
+  const int tile = verify_tile(rows, value_heads, K, V, E == 4, qm, pending != nullptr);
   a.NVT = int32_t((V + tile - 1) / tile);
   a.nvt_magic = udiv_magic(uint32_t(a.NVT));
   if (int64_t(a.NVT) * value_heads > 0x7fffffffLL) {
