@@ -105,6 +105,7 @@ __host__ __device__ inline uint32_t udiv(uint32_t x, uint32_t d, uint32_t m) {
 constexpr int kVerifyThreads = 64;  // one wave per (row, value head, tile)
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <typename A>
 __device__ __forceinline__ void st_f32_or(void *p, int64_t i, bool f32, float x) {
@@ -288,9 +289,32 @@ __device__ __forceinline__ float sum_blocks(float x) {
   x = swap_add16(x, x);
   return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
 }
-__device__ __forceinline__ float sum_quarters(float x) {  // over the lanes of equal l % 16
-  x = swap_add32(x, x);
-  return swap_add16(x, x);
+// WIDE: the sum over a row's chunks c = 4j + quarter of a value per chunk, in the
+// order of sum_blocks (c ^ 8, c ^ 4, c ^ 2, c ^ 1).
+template <int CJ>
+__device__ __forceinline__ float sum_chunks(const float (&x)[CJ]) {
+  float y;
+  if constexpr (CJ == 4)
+    y = (x[0] + x[2]) + (x[1] + x[3]);
+  else
+    y = x[0] + x[1];
+  y = swap_add32(y, y);
+  return swap_add16(y, y);
+}
+// The same of CJ 16x16x1 results, register 4*(c % 4) + r: register r of the sum.
+template <int CJ, typename F>
+__device__ __forceinline__ f32x4 sum_results(const F &product) {  // product(j): the result of chunks 4j .. 4j + 3
+  f32x16 x;
+  if constexpr (CJ == 4) {
+    x = product(0) + product(2);
+    x += product(1) + product(3);
+  } else {
+    x = product(0) + product(1);
+  }
+  f32x4 y;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) y[r] = (x[r] + x[8 + r]) + (x[4 + r] + x[12 + r]);
+  return y;
 }
 // The sum for the four registers of a 4x4 result tile at once. N = 16: lane
 // 16*r + 4*any + i gets the sum of row r, column i. N = 8: `lo` gets rows 0 (lanes
@@ -316,7 +340,7 @@ __device__ __forceinline__ void reduce_rows8(f32x4 a, float &lo, float &hi) {
 template <int QM, int KP, bool DEFER, int TILE, int STAGE>
 struct __align__(16) VerifyLds {
   static constexpr int HALF = TILE < 64 ? TILE : 64;
-  uint4 stage[STAGE];         // one block of rows on its way to the 16x16x4 layout
+  uint4 stage[STAGE];         // one block of rows on its way to the 16x16x1 layout
   float d[HALF][2 * QM + 1];  // GEMV results of one half tile
   __align__(16) float pk[DEFER ? QM : 1][DEFER ? KP : 1];  // pending commit's keys
   float pc[DEFER ? QM : 1][DEFER ? HALF : 1];              // and its corrections of the tile's rows
@@ -332,17 +356,19 @@ __host__ __device__ constexpr int verify_block_rows(int qm) {
   return sizeof(S) == 4 && KP == 256 && qm == 8 ? 8 : 16;
 }
 
-// Windows of more than four tokens have 16 columns, a whole 16x16x4 instruction:
-// the same matrix-core time as 4x4x1 ones and no cross-lane sums, which are ten
-// instructions per four rows and four columns. Tiles of 64 rows and up whose rows
-// are at most 256 bytes are bound by instructions there, so their blocks go
-// through LDS into that layout (lane l holds row l % 16, chunks 4j + l / 16): one
-// write and one read per load of 1 KiB. One layer of 32 heads, Q = 8, us with 4x4x1
-// / 16x16x4: FP16 K = 128, V = 128, 64 rows 34.4 / 28.4, 256 rows 108 / 89; FP16 K = 64,
-// V = 192, 256 rows 103 / 82; BF16 K = 64, V = 128, 256 rows 68 / 58; FP32 K = 64, V =
-// 128, 32 rows 18.8 / 16.0, 256 rows 81 / 75. Tiles of 16 rows are a chain of
-// latencies that the detour lengthens (BF16 K = 128, 4 rows 7.4 / 9.0), and the
-// deferred verify is bound by its fold (BF16 K = 128, 64 rows 54.6 / 58.0).
+// Windows of more than four tokens have 16 columns: a 16x16x1 instruction of four
+// blocks (one per quarter of the wave) takes the same matrix-core time as 4x4x1
+// ones, and its partial sums meet in a lane's own registers, 60 adds per 16 rows
+// instead of 160 cross-lane instructions. Tiles of 64 rows and up whose rows are at
+// most 256 bytes are bound by instructions there, so their blocks go through LDS
+// into that layout (lane l holds row l % 16, chunks 4j + l / 16): one write and one
+// read per load of 1 KiB. Products and sums keep the 4x4x1 form's order, so that a
+// row's result does not depend on the launch it is in. One layer of 32 heads, Q = 8,
+// us with 4x4x1 / 16x16x1: FP16 K = V = 128, 64 rows 34.4 / 29.5, 256 rows 108 / 91; FP16
+// K = 64, V = 192, 256 rows 103 / 85; BF16 K = 64, V = 128, 256 rows 68 / 61; FP32 K = 64,
+// V = 128, 32 rows 18.8 / 15.4, 256 rows 81 / 75. Tiles of 16 rows are a chain of latencies
+// that the detour lengthens (BF16 K = 128, 4 rows 7.4 / 9.0), and the deferred verify is
+// bound by its fold (BF16 K = 128, 64 rows 54.6 / 58.0).
 template <typename S, int KP>
 __host__ __device__ constexpr bool verify_wide(int qm, bool defer, int tile) {
   return qm == 8 && !defer && tile >= 64 && KP * int(sizeof(S)) <= 256;
@@ -687,12 +713,17 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
     // kernels.py:645-648: x * rsqrt(sum(x*x) + 1e-6) for q and k, then q *= scale.
 #pragma unroll
     for (int cg = 0; cg < CG; ++cg) {
-      float ss = 0.0f;
+      float ss[CJ] = {};  // WIDE: of each chunk
 #pragma unroll
       for (int j = 0; j < CJ; ++j)
 #pragma unroll
-        for (int e = 0; e < E; ++e) ss = __builtin_fmaf(m[cg][j][e], m[cg][j][e], ss);
-      const float inv = rsqrtf((WIDE ? sum_quarters(ss) : sum_blocks<R::N>(ss)) + 1e-6f);
+        for (int e = 0; e < E; ++e) ss[WIDE ? j : 0] = __builtin_fmaf(m[cg][j][e], m[cg][j][e], ss[WIDE ? j : 0]);
+      float total;
+      if constexpr (WIDE)
+        total = sum_chunks(ss);
+      else
+        total = sum_blocks<R::N>(ss[0]);
+      const float inv = rsqrtf(total + 1e-6f);
 #pragma unroll
       for (int j = 0; j < CJ; ++j)
 #pragma unroll
@@ -741,15 +772,12 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
   float gram[WIDE ? 1 : CGK][WIDE ? 1 : CG];
   f32x4 wide_gram = {0.0f, 0.0f, 0.0f, 0.0f};
   if constexpr (WIDE) {
-    f32x4 odd = {0.0f, 0.0f, 0.0f, 0.0f};
+    wide_gram = sum_results<CJ>([&](int j) {
+      f32x16 acc = {};
 #pragma unroll
-    for (int j = 0; j < CJ; ++j)
-#pragma unroll
-      for (int e = 0; e < E; e += 2) {
-        wide_gram = __builtin_amdgcn_mfma_f32_16x16x4f32(m[0][j][e], m[0][j][e], wide_gram, 0, 0, 0);
-        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(m[0][j][e + 1], m[0][j][e + 1], odd, 0, 0, 0);
-      }
-    wide_gram += odd;
+      for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(m[0][j][e], m[0][j][e], acc, 0, 0, 0);
+      return acc;
+    });
   } else {
 #pragma unroll
     for (int s = 0; s < CGK; ++s)
@@ -887,15 +915,13 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
     uint4 op[CJ];
 #pragma unroll
     for (int j = 0; j < CJ; ++j) op[j] = L.stage[stage_slot(cl, 4 * j + cs)];
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, odd = acc;
+    const f32x4 acc = sum_results<CJ>([&](int j) {
+      f32x16 x = {};
 #pragma unroll
-    for (int j = 0; j < CJ; ++j)
-#pragma unroll
-      for (int e = 0; e < E; e += 2) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(chunk_elem<S>(op[j], e), m[0][j][e], acc, 0, 0, 0);
-        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(chunk_elem<S>(op[j], e + 1), m[0][j][e + 1], odd, 0, 0, 0);
-      }
-    acc += odd;
+      for (int e = 0; e < E; ++e)
+        x = __builtin_amdgcn_mfma_f32_16x16x1f32(chunk_elem<S>(op[j], e), m[0][j][e], x, 0, 0, 0);
+      return x;
+    });
     const int row = (rb & (HRB - 1)) * BROWS + 4 * cs;
 #pragma unroll
     for (int i = 0; i < 4; ++i) d_lds[row + i][cl] = acc[i];
@@ -1043,16 +1069,18 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
 // buffers and the B operands take at most 96 registers; past that (FP32 pages of
 // K > 128, 16-bit ones at Q > 4) three waves spilled, and the bound is two (K =
 // 256, 32 heads of V = 128, us with three waves / two: FP32 pages Q = 4, 128 rows
-// 152 / 103, Q = 1 99 / 90; BF16 pages Q = 8, 128 rows 100 / 94).
-template <typename S, int KP>
+// 152 / 103, Q = 1 99 / 90; BF16 pages Q = 8, 128 rows 100 / 94). So it is where FP32
+// activations meet the 16x16x1 form's accumulators on rows of 128 16-bit elements.
+template <typename S, typename A, int KP>
 constexpr int verify_min_waves(int qm, int tile) {
   using R = RowLanes<S, KP>;
   const int buffers = 2 * (verify_block_rows<S, KP>(qm) / R::ROWS) * R::J * 4;
   const int operands = (2 * qm + 3) / 4 * R::J * R::E;
-  return tile < 128 ? 1 : buffers + operands <= 96 ? 3 : 2;
+  const bool wide_f32 = verify_wide<S, KP>(qm, false, tile) && KP == 128 && sizeof(A) == 4;
+  return tile < 128 ? 1 : buffers + operands <= 96 && !wide_f32 ? 3 : 2;
 }
 template <typename S, typename A, int KP, int QM, bool DEFER, int TILE>
-__global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, KP>(QM, TILE))) void verify_kernel(VerifyArgs a) {
+__global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, A, KP>(QM, TILE))) void verify_kernel(VerifyArgs a) {
   __shared__ VerifyLds<QM, KP, DEFER, TILE, verify_stage<S, KP>(QM, DEFER, TILE)> lds;
   warm_kernel_args<int(sizeof(VerifyArgs))>();
   if (DEFER || int(blockIdx.y) < a.nt_rows)  // the deferred verify: every row (see verify.hip)
