@@ -46,6 +46,8 @@
 // QM window capacity (Q <= QM).
 #pragma once
 
+#include <type_traits>
+
 #include "gdn_common.cuh"
 
 namespace gdn {
@@ -270,9 +272,12 @@ struct RowLanes {
 
 // The sum over a row's N blocks (16: all of kb = lane / 4, 8: kb % 8) of a value
 // per (block, lane % 4), in every lane of the row.
+// A rotation has no lane without a source, and the last argument says so: with
+// false the compiler keeps the move apart from the add (FP32 K = V = 128, Q = 4, 32
+// heads, 1 row 5.3 us, folded 4.9).
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float x) {
-  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
+  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
 }
 constexpr int kRowRor8 = 0x128, kRowRor4 = 0x124;  // rotations inside 16 lanes
 __device__ __forceinline__ float swap_add32(float x, float y) {  // lanes 0-31: x summed over the halves; 32-63: y
@@ -1071,16 +1076,23 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
 // 256, 32 heads of V = 128, us with three waves / two: FP32 pages Q = 4, 128 rows
 // 152 / 103, Q = 1 99 / 90; BF16 pages Q = 8, 128 rows 100 / 94). So it is where FP32
 // activations meet the 16x16x1 form's accumulators on rows of 128 16-bit elements.
+// Shorter tiles at Q > 4 ask for two waves, which leaves a wave 256 registers and
+// none of the accumulation file: with one, every product was copied out of it
+// (FP32 K = 64, V = 192, Q = 8, 256 rows 122 / 113 us; K = V = 128, deferred, 64 rows
+// 71 / 68); the deferred FP16 kernels of K > 128 do not fit. At Q <= 4 the choice
+// made no difference but at K = 256, where one is faster (1 row 6.2 / 6.7).
 template <typename S, typename A, int KP>
-constexpr int verify_min_waves(int qm, int tile) {
+constexpr int verify_min_waves(int qm, int tile, bool defer) {
   using R = RowLanes<S, KP>;
   const int buffers = 2 * (verify_block_rows<S, KP>(qm) / R::ROWS) * R::J * 4;
   const int operands = (2 * qm + 3) / 4 * R::J * R::E;
-  const bool wide_f32 = verify_wide<S, KP>(qm, false, tile) && KP == 128 && sizeof(A) == 4;
-  return tile < 128 ? 1 : buffers + operands <= 96 && !wide_f32 ? 3 : 2;
+  const bool wide_f32 = verify_wide<S, KP>(qm, defer, tile) && KP == 128 && sizeof(A) == 4;
+  if (tile == 128) return buffers + operands <= 96 && !wide_f32 ? 3 : 2;
+  return qm == 8 && !(defer && KP == 256 && std::is_same_v<S, f16>) ? 2 : 1;
 }
 template <typename S, typename A, int KP, int QM, bool DEFER, int TILE>
-__global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, A, KP>(QM, TILE))) void verify_kernel(VerifyArgs a) {
+__global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, A, KP>(QM, TILE, DEFER))) void verify_kernel(
+    VerifyArgs a) {
   __shared__ VerifyLds<QM, KP, DEFER, TILE, verify_stage<S, KP>(QM, DEFER, TILE)> lds;
   warm_kernel_args<int(sizeof(VerifyArgs))>();
   if (DEFER || int(blockIdx.y) < a.nt_rows)  // the deferred verify: every row (see verify.hip)
