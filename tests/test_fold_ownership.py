@@ -7,9 +7,9 @@ kernels that write state pages in place:
   ``tid // KCH + pass * RP``; passes go in batches of ``64 / E`` loads, each
   batch's stores after its loads;
 * the deferred verify (csrc/verify_kernel.cuh, ``DEFER``): one wave per
-  (row, value head, 64-row half tile); block ``rb``'s stores (final page and
-  boundary snapshot) come after its loads, and the loads of block ``rb + 2``
-  after those stores.
+  (row, value head, tile of 16, 32 or 64 rows); block ``rb``'s stores (final
+  page and boundary snapshot) come after its loads, and the loads of block
+  ``rb + 2`` after those stores.
 
 A row's source, final and boundary pages may be one page (the plan makes
 ``boundary == source`` whenever the window crosses a block boundary from the
@@ -136,51 +136,61 @@ def test_alias_case_known_answer_and_the_double_fold():
     assert bad == 2.25
 
 
-def _defer_events(K, V, E, vs, J, rounds):
-    """The deferred verify's non-temporal body for one tile: wave vt covers
-    rows [64 vt, 64 vt + 64); block rb's 16 rows are loaded as row runs
-    (load j: rows (j % JR) * RPL + lane // SC, chunks (j // JR) * SC + lane % SC)
-    and stored back with the same offsets after its fold; blocks rb and
-    rb + 1 are in flight together, rb + 2 is loaded after rb's stores."""
-    cpr = 4 * J
-    SC, JR = cpr // rounds, J // rounds
-    RPL = 64 // SC
+def _defer_events(K, V, E, vs, tile, block=16):
+    """The deferred verify for one (row, value head): wave vt covers rows
+    [tile * vt, tile * vt + tile) in blocks; register g*J + j of a block is
+    loaded, and stored back after its fold, at row ROWS*g + lr, chunk N*j + kb
+    (RowLanes: a row over N = 16 blocks of four lanes, over 8 for up to 64
+    16-bit elements). Blocks rb and rb + 1 are in flight together, rb + 2 is
+    loaded after rb's stores. Chunks past K get an out-of-range offset, rows
+    past V lie outside the tile's resource of tile_rows * vs elements."""
+    kp = 64 if K <= 64 else 128 if K <= 128 else 256
+    N = 8 if E == 8 and kp == 64 else 16
+    J, rows_per_load = kp // (N * E), 64 // N
     events = []
-    nvt = -(-V // 64)
-    for vt in range(nvt):
-        row0 = vt * 64
-        tile_rows = min(64, V - row0)
+    for vt in range(-(-V // tile)):
+        row0 = vt * tile
+        tile_rows = min(tile, V - row0)
 
-        def block(rb):
+        def accesses(rb):
             out = []
-            for j in range(J):
-                for lane in range(64):
-                    r = rb * 16 + (j % JR) * RPL + lane // SC
-                    c = (j // JR) * SC + lane % SC
-                    if c * E < K and r < tile_rows:
-                        out.append((lane, (row0 + r, c)))
+            for g in range(block // rows_per_load):
+                for j in range(J):
+                    for lane in range(64):
+                        kb, ij = (lane >> 2) & (N - 1), lane & 3
+                        lr = ij if N == 16 else 4 * (lane >> 5) + ij
+                        r, c = rb * block + rows_per_load * g + lr, N * j + kb
+                        if c * E < K and r * vs + c * E < tile_rows * vs:
+                            out.append((lane, (row0 + r, c)))
             return out
 
-        order = [("load", 0), ("load", 1)]
-        for rb in range(4):
+        blocks = tile // block
+        order = [("load", rb) for rb in range(min(2, blocks))]
+        for rb in range(blocks):
             order.append(("store", rb))
-            if rb + 2 < 4:
+            if rb + 2 < blocks:
                 order.append(("load", rb + 2))
         for kind, rb in order:
-            for lane, ch in block(rb):
+            for lane, ch in accesses(rb):
                 events.append((vt, lane, 0, kind, ch))
     return events
 
 
-@pytest.mark.parametrize("K,V,E,J", [(128, 128, 4, 8), (128, 128, 8, 4), (256, 256, 4, 16), (64, 96, 4, 4),
-                                     (16, 8, 4, 1), (32, 128, 4, 2)])
-@pytest.mark.parametrize("rounds", [1, 2, 4])
-def test_deferred_verify_tile_has_one_owner_per_chunk(K, V, E, J, rounds):
-    """For any number of staging rounds that divides the block's loads."""
-    if J % rounds or 64 % (4 * J // rounds):
-        pytest.skip("not a staging of this J")
-    assert 4 * E * J >= K
-    assert _check_single_owner(_defer_events(K, V, E, K, J, rounds), K, V, E) is None
+@pytest.mark.parametrize("K,E", [(128, 4), (128, 8), (256, 4), (256, 8), (64, 4), (64, 8), (8, 8), (16, 4), (96, 4),
+                                 (136, 8)])
+@pytest.mark.parametrize("V", [128, 96, 40, 17, 8])
+@pytest.mark.parametrize("tile", [16, 32, 64])
+def test_deferred_verify_tile_has_one_owner_per_chunk(K, V, E, tile):
+    for block in (16, 8) if E == 4 and K > 128 else (16,):  # 8-row blocks: FP32 pages of K > 128 at Q > 4
+        assert _check_single_owner(_defer_events(K, V, E, K, tile, block), K, V, E) is None
+
+
+def test_overlapping_deferred_tiles_break_the_single_owner_rule():
+    """Tiles that advance by less than their rows share chunks."""
+    events = _defer_events(128, 64, 4, 128, 32)
+    moved = [(wg, lane, b, kind, (r - 16 * wg, c)) for wg, lane, b, kind, (r, c) in events]
+    problem = _check_single_owner(moved, 128, 48, 4)
+    assert problem is not None and "twice" in problem
 
 
 def test_plan_outputs_never_feed_the_fused_launch():

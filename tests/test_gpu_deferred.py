@@ -332,8 +332,9 @@ def test_deferred_commit_equals_ordinary_flow(dev, seed, empty_row):
 ])
 def test_deferred_commit_equals_ordinary_flow_shapes(dev, K, V, Q, H, HV, act, state):
     """The same equality over head dims off the 128 x 128 tile (partial
-    64-row half tiles, K padded to whole chunks), windows 1-8, GQA ratios 1-4,
-    every activation dtype and every state dtype."""
+    tiles of 16 rows, K padded to whole chunks), windows 1-8, GQA ratios 1-4,
+    every activation dtype and every state dtype. Longer tiles:
+    test_gpu_verify_batch_bits.py."""
     steps = 3
     w = W.make_workload("decode_loop_l48", layers=2, rows=6, key_heads=H, value_heads=HV, key_dim=K, value_dim=V,
                         window=Q, act_dtype=act, state_dtype=state, steps=steps, max_position=256, block_size=8,

@@ -30,7 +30,7 @@ EXTREMES = {
     # many rows with small heads: 2048 rows, 2 value heads of 32 x 32, Q=2
     "rows_2048": ("pool512_b64", dict(rows=2048, key_heads=1, value_heads=2, key_dim=32, value_dim=32, window=2,
                                       pool_pages=2100)),
-    # the largest heads the kernels take: K=256, V=1024 (eight verify tiles), Q=8, align mode
+    # the largest heads the kernels take: K=256, V=1024 (384 waves of 16 rows), Q=8, align mode
     "k256_v1024_q8": ("align_b256", dict(rows=3, key_heads=1, value_heads=2, key_dim=256, value_dim=1024, window=8,
                                          padded_rows=0, crossing_fraction=1.0)),
 }

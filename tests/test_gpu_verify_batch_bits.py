@@ -88,6 +88,9 @@ def test_deferred_tiles_equal_the_ordinary_flow(dev, Q, K, V, state, act):
         gen = torch.Generator().manual_seed(K * V + Q)
         acc_steps = [W.sample_accepted(w.spec, rows, gen) for _ in range(steps)]
         qsl_steps = [w.meta.query_start_loc.clone() for _ in range(steps)]
+        lens = torch.full((rows,), Q, dtype=torch.int32)
+        lens[rows // 2] = 0  # a row with nothing to verify, its commit pending
+        qsl_steps[-1][1:] = torch.cumsum(lens, 0)
         ref = _flow(w, dev, acc_steps, qsl_steps, deferred=False)
         _assert_flows_equal(ref, _flow(w, dev, acc_steps, qsl_steps, deferred=True))
     assert seen - {16}

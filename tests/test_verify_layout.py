@@ -1,69 +1,52 @@
-"""The verify's LDS staging of non-temporal state blocks (csrc/verify_kernel.cuh,
-`row_slot` / `op_slot` and the loads' `c_voff` / `c_soff`), restated on the CPU
-for every chunk count J the kernel is instantiated with. A block is 16 rows x
-CPR = 4J chunks of 16 bytes, staged in ROUNDS rounds of SC = CPR / ROUNDS
-chunks per row (two rounds for J >= 2). Load j (round g = j // JR) gives lane
-l the chunk (row (j % JR) * RPL + l // SC, chunk g * SC + l % SC) and writes
-it to slot r * SC + (c ^ swz(r)) of its round; operand register j of lane
-(li, ls) reads chunk 4j + ls of row li back. Checked: every operand register
-receives exactly the chunk the matrix-core layout assigns it (the layout the
-ordinary loads produce directly), the loads cover the block once in runs of
-SC consecutive chunks, each write covers 64 consecutive slots, and the 16
-lanes of a read that share ls hit 16 distinct 16-byte bank groups. The GPU
-tests compare the two load bodies' results bit for bit."""
+"""The verify's LDS staging of the 16x16x1 form (csrc/verify_kernel.cuh, `stage_slot`,
+`stage_block` and `wide_block`), restated on the CPU for the chunk counts it is
+instantiated with: rows of CPR = 16 chunks of 16 bytes (256 bytes) loaded over N = 16
+blocks, and of CPR = 8 (64 16-bit elements) over N = 8. A block is 16 rows; load g
+gives lane l the chunk kb of row ROWS*g + lr and writes it to slot r*CPR +
+(c ^ swz(r)); operand register j of lane l reads chunk 4j + l / 16 of row l % 16 back.
+Checked: every operand register receives exactly the chunk the matrix-core layout
+assigns it, the loads cover the block once, and the 16 lanes of each quarter of a
+write, and the 16 rows a read takes of one chunk, hit 16 distinct 16-byte bank
+groups. The GPU tests compare the form's results with the 4x4x1 form's bit for bit."""
 
 import pytest
 
 
-def _geometry(J):
-    cpr = 4 * J
-    rounds = 2 if J >= 2 else 1
-    sc = cpr // rounds
-    jr = J // rounds
-    rpl = 64 // sc
-    mask = (sc if sc < 16 else 16) - 1
-    sh = 0 if sc >= 16 else (1 if sc == 8 else 2)
-    return cpr, rounds, sc, jr, rpl, (lambda r: (r >> sh) & mask)
+def _geometry(cpr):
+    n = cpr  # blocks (of four lanes) that share a row
+    rows = 64 // n
+    swz = (lambda r: ((r & 3) << 2) | (r >> 2)) if cpr == 16 else (lambda r: ((r & 2) << 1) | (r >> 2))
+    return n, rows, lambda r, c: r * cpr + (c ^ swz(r))
 
 
-@pytest.mark.parametrize("J", [1, 2, 4, 8, 16])
-def test_staging_rounds_map_row_runs_to_the_operand_layout(J):
-    cpr, rounds, sc, jr, rpl, swz = _geometry(J)
-    assert rounds * jr == J and sc == 4 * jr
-    for g in range(rounds):
-        stage = {}
-        for j in range(g * jr, (g + 1) * jr):
-            slots = set()
-            for lane in range(64):
-                r, c = (j % jr) * rpl + lane // sc, lane % sc
-                assert r < 16
-                slot = r * sc + (c ^ swz(r))
-                assert slot not in stage
-                stage[slot] = (r, g * sc + c)
-                slots.add(slot)
-            jj = j % jr
-            assert slots == set(range(64 * jj, 64 * jj + 64)), "a write must cover 64 consecutive slots"
-        assert len(stage) == 16 * sc, "a round's stage must be filled exactly once"
-        for j in range(g * jr, (g + 1) * jr):
-            for ls in range(4):
-                groups = set()
-                for li in range(16):
-                    slot = li * sc + ((4 * (j % jr) + ls) ^ swz(li))
-                    assert stage[slot] == (li, 4 * j + ls), "operand register got another chunk"
-                    groups.add(slot % 16)
-                assert len(groups) == 16, "bank conflict among the lanes of one read"
+def _written(cpr, g):
+    """(row, chunk) of each lane of load g."""
+    n, rows, _ = _geometry(cpr)
+    return [(rows * g + (lane & 3 if n == 16 else 4 * (lane >> 5) + (lane & 3)), (lane >> 2) & (n - 1))
+            for lane in range(64)]
 
 
-@pytest.mark.parametrize("J", [1, 2, 4, 8, 16])
-def test_row_run_loads_cover_the_block_once(J):
-    """Every chunk of a 16-row block is loaded once; each load reads SC
-    consecutive chunks of each of its rows (row-major within the round)."""
-    cpr, rounds, sc, jr, rpl, _ = _geometry(J)
-    seen = []
-    for j in range(J):
-        g = j // jr
-        offs = [((j % jr) * rpl + lane // sc) * cpr + g * sc + lane % sc for lane in range(64)]
-        for k in range(0, 64, sc):
-            assert offs[k:k + sc] == list(range(offs[k], offs[k] + sc))
-        seen += offs
-    assert sorted(seen) == list(range(16 * cpr))
+@pytest.mark.parametrize("cpr", [16, 8])
+def test_staging_maps_row_runs_to_the_operand_layout(cpr):
+    _, rows, slot = _geometry(cpr)
+    stage = {}
+    for g in range(16 // rows):
+        at = [slot(r, c) for r, c in _written(cpr, g)]
+        for lane, rc in enumerate(_written(cpr, g)):
+            assert at[lane] not in stage
+            stage[at[lane]] = rc
+        for quarter in range(0, 64, 16):
+            assert len({x % 16 for x in at[quarter:quarter + 16]}) == 16, "bank conflict in a write"
+    assert sorted(stage) == list(range(16 * cpr)), "the stage must be filled exactly once"
+    for j in range(cpr // 4):
+        for quarter in range(4):
+            at = [slot(row, 4 * j + quarter) for row in range(16)]
+            assert [stage[x] for x in at] == [(row, 4 * j + quarter) for row in range(16)]
+            assert len({x % 16 for x in at}) == 16, "bank conflict among the lanes of one read"
+
+
+@pytest.mark.parametrize("cpr", [16, 8])
+def test_row_run_loads_cover_the_block_once(cpr):
+    _, rows, _ = _geometry(cpr)
+    seen = [rc for g in range(16 // rows) for rc in _written(cpr, g)]
+    assert sorted(seen) == [(r, c) for r in range(16) for c in range(cpr)]

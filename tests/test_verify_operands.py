@@ -133,27 +133,27 @@ def test_runs_of_16_bit_elements(N, first):
     assert out == elems[first:first + N]
 
 
-@pytest.mark.parametrize("cpr,N,rows", [(16, 16, 4), (8, 8, 8)])
-def test_stage_slots(cpr, N, rows):
-    """The staged block of the 16x16x4 form: one slot per chunk; the 16 lanes of a
-    quarter of a write, and the 16 rows a read takes of one chunk, in 16 places
-    modulo 256 bytes; a read gives lane l row l % 16, chunk 4j + l / 16."""
-    def slot(row, c):
-        return row * cpr + (c ^ (((row & 3) << 2) | (row >> 2) if cpr == 16 else ((row & 2) << 1) | (row >> 2)))
+@pytest.mark.parametrize("chunks", [16, 8])
+def test_both_forms_sum_the_chunks_in_one_order(chunks):
+    """The tree of reduce_rows / reduce_rows8 over a row's chunks (kb ^ 8, ^ 4, ^ 2, ^ 1
+    by lane) and of sum_results (chunk 4j + block: j, then block ^ 2, ^ 1) add the
+    same pairs at every level, so the two give the same bits."""
+    def pair(level, bit):
+        return {c: frozenset((level[c], level[c ^ bit])) for c in level}
 
-    stage = {}
-    for g in range(16 // rows):
-        at = []
-        for lane in range(64):
-            kb, ij = (lane >> 2) & (N - 1), lane & 3
-            row = rows * g + (ij if N == 16 else 4 * (lane >> 5) + ij)
-            at.append(slot(row, kb))
-            assert at[-1] not in stage
-            stage[at[-1]] = (row, kb)
-        assert all(len({x % 16 for x in at[q:q + 16]}) == 16 for q in range(0, 64, 16))
-    assert sorted(stage) == list(range(16 * cpr))
-    for j in range(cpr // 4):
-        for s in range(4):
-            at = [slot(row, 4 * j + s) for row in range(16)]
-            assert [stage[x] for x in at] == [(row, 4 * j + s) for row in range(16)]
-            assert len({x % 16 for x in at}) == 16
+    lanes = {c: c for c in range(chunks)}
+    for bit in ([8] if chunks == 16 else []) + [4, 2, 1]:
+        lanes = pair(lanes, bit)
+
+    def product(j):
+        return {b: 4 * j + b for b in range(4)}
+
+    def add(x, y):
+        return {b: frozenset((x[b], y[b])) for b in x}
+
+    if chunks == 16:
+        x = add(add(product(0), product(2)), add(product(1), product(3)))
+    else:
+        x = add(product(0), product(1))
+    got = frozenset((frozenset((x[0], x[2])), frozenset((x[1], x[3]))))
+    assert all(v == got for v in lanes.values())
