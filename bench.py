@@ -184,8 +184,8 @@ def _probe_lib():
 
 def _verify_twin(lib, w, layer, nbytes, retain):
     """The verify twin of one layer's launch: its state tiles (the rows before
-    the last ``retain`` bytes non-temporally in row runs, the rest in the
-    operand layout, as the verify reads them), its small reads and its output
+    the last ``retain`` bytes non-temporally, the rest with ordinary loads,
+    all in row runs, as the verify reads them), its small reads and its output
     and record writes. Returns (launch, launch without the small traffic,
     bytes moved, tiles)."""
     import torch
@@ -307,7 +307,7 @@ def traffic_ceiling(w, nbytes, plan, kernel_us, timer, steps, retain=None):
                 "(verify twin: the verify's state tiles, small reads and output / record writes; fold twin: the "
                 "committed tiles copied to their final and boundary pages of a scratch pool), timed as a step; "
                 "reads_only: the verify twin without its small reads and writes; the verify twin reads the tiles "
-                "of the rows before the last retained bytes non-temporally in row runs, as the verify does",
+                "in row runs, those of the rows before the last retained bytes non-temporally, as the verify does",
     }
 
 

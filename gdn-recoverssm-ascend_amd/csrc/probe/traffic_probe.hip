@@ -21,16 +21,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const char *p, int b
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(p), 0, bytes, 0x00020000);
 }
 
-// The verify's traffic: one wave per tile; `small_dw` dwords read from a
-// region two consecutive waves share (q and k are shared by the two value
-// heads of a key head); the tile streamed as eight 16-row blocks, two blocks
-// in flight; `write_dw` dwords written per wave, half after each 64-row half
-// tile, as the verify stores its outputs and records. Tiles w < nt_tiles read
-// row runs with non-temporal loads (lane l, load j: row 4 (j % 4) + l / 16,
-// 16-byte chunk 16 (j / 4) + l % 16 of the block: 4 rows x 256 bytes), the
-// rest the matrix-core operand layout with ordinary loads (lane (r = l % 16,
-// s = l / 16) reads the 16-byte chunks 4j + s of row r), as the verify's two
-// bodies do.
+// The verify's traffic: one wave per tile of 128 rows (the tile that large
+// launches take); `small_dw` dwords read from a region two consecutive waves
+// share (q and k are shared by the two value heads of a key head); the tile
+// streamed as eight 16-row blocks, two blocks in flight; `write_dw` dwords
+// written per wave, half after each 64-row half tile, as the verify stores its
+// outputs and records. Every load reads row runs in the verify's lane layout
+// (lane l, load j: row 4 (j % 4) + l % 4, 16-byte chunk 16 (j / 4) + l / 4 of the
+// block: 4 rows x 256 bytes); tiles w < nt_tiles with non-temporal loads, the
+// rest with ordinary ones.
 template <bool NT>
 __device__ __forceinline__ float verify_twin_tile(__amdgpu_buffer_rsrc_t r, __amdgpu_buffer_rsrc_t wr, int lane,
                                                   int write_dw, float acc) {
@@ -38,8 +37,7 @@ __device__ __forceinline__ float verify_twin_tile(__amdgpu_buffer_rsrc_t r, __am
   int voff[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j)
-    voff[j] = NT ? ((j & 3) * 4 + (lane >> 4)) * kRowBytes + ((j >> 2) * 16 + (lane & 15)) * 16
-                 : (lane & 15) * kRowBytes + (4 * j + (lane >> 4)) * 16;
+    voff[j] = ((j & 3) * 4 + (lane & 3)) * kRowBytes + ((j >> 2) * 16 + (lane >> 2)) * 16;
   u32x4 a[8], b[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) a[j] = __builtin_amdgcn_raw_buffer_load_b128(r, voff[j], 0, pol);
