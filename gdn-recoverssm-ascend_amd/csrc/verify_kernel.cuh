@@ -272,12 +272,11 @@ struct RowLanes {
 
 // The sum over a row's N blocks (16: all of kb = lane / 4, 8: kb % 8) of a value
 // per (block, lane % 4), in every lane of the row.
-// A rotation has no lane without a source, and the last argument says so: with
-// false the compiler keeps the move apart from the add (FP32 K = V = 128, Q = 4, 32
-// heads, 1 row 5.3 us, folded 4.9).
-template <int CTRL>
+// A rotation has no lane without a source. FOLD says so, and the move becomes part
+// of the add (FP32 K = V = 128, Q = 4, 8 rows 8.6 / 8.3 us); see verify_wave for where not.
+template <int CTRL, bool FOLD>
 __device__ __forceinline__ float dpp_add(float x) {
-  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, FOLD));
 }
 constexpr int kRowRor8 = 0x128, kRowRor4 = 0x124;  // rotations inside 16 lanes
 __device__ __forceinline__ float swap_add32(float x, float y) {  // lanes 0-31: x summed over the halves; 32-63: y
@@ -288,11 +287,11 @@ __device__ __forceinline__ float swap_add16(float x, float y) {  // even 16-lane
   const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
   return __uint_as_float(p[0]) + __uint_as_float(p[1]);
 }
-template <int N>
+template <int N, bool FOLD>
 __device__ __forceinline__ float sum_blocks(float x) {
   if constexpr (N == 16) x = swap_add32(x, x);
   x = swap_add16(x, x);
-  return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
+  return dpp_add<kRowRor4, FOLD>(dpp_add<kRowRor8, FOLD>(x));
 }
 // WIDE: the sum over a row's chunks c = 4j + quarter of a value per chunk, in the
 // order of sum_blocks (c ^ 8, c ^ 4, c ^ 2, c ^ 1).
@@ -324,13 +323,15 @@ __device__ __forceinline__ f32x4 sum_results(const F &product) {  // product(j):
 // The sum for the four registers of a 4x4 result tile at once. N = 16: lane
 // 16*r + 4*any + i gets the sum of row r, column i. N = 8: `lo` gets rows 0 (lanes
 // of even 16) and 1 (odd), `hi` rows 2 and 3, each half of the wave its own tile.
+template <bool FOLD>
 __device__ __forceinline__ float reduce_rows(f32x4 a) {
   const float x = swap_add16(swap_add32(a[0], a[2]), swap_add32(a[1], a[3]));
-  return dpp_add<kRowRor4>(dpp_add<kRowRor8>(x));
+  return dpp_add<kRowRor4, FOLD>(dpp_add<kRowRor8, FOLD>(x));
 }
+template <bool FOLD>
 __device__ __forceinline__ void reduce_rows8(f32x4 a, float &lo, float &hi) {
-  lo = dpp_add<kRowRor4>(dpp_add<kRowRor8>(swap_add16(a[0], a[1])));
-  hi = dpp_add<kRowRor4>(dpp_add<kRowRor8>(swap_add16(a[2], a[3])));
+  lo = dpp_add<kRowRor4, FOLD>(dpp_add<kRowRor8, FOLD>(swap_add16(a[0], a[1])));
+  hi = dpp_add<kRowRor4, FOLD>(dpp_add<kRowRor8, FOLD>(swap_add16(a[2], a[3])));
 }
 
 // DEFER: before verifying, apply the previous step's commit for this row (the
@@ -396,6 +397,9 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
   constexpr int CGK = (QM + CW - 1) / CW;      // column groups that hold a k
   constexpr int CN = WIDE ? 4 : R::N;          // lanes that share a column's vector
   constexpr int CJ = KP / (CN * E);            // chunks of it per lane
+  // Rotated adds as one instruction, but in the kernel whose scalars the compiler
+  // then spills around every block (K = 256, 32 heads, 1 row 6.2 us, folded 6.7).
+  constexpr bool FOLD = !(sizeof(S) == 4 && KP == 256 && QM == 4 && TILE == 16 && !DEFER);
   constexpr bool MIXED = QM % CW != 0;         // a group may hold k and q columns
   constexpr int BROWS = verify_block_rows<S, KP>(QM);
   constexpr int BG = BROWS / R::ROWS;  // loads of a block per chunk
@@ -727,7 +731,7 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
       if constexpr (WIDE)
         total = sum_chunks(ss);
       else
-        total = sum_blocks<R::N>(ss[0]);
+        total = sum_blocks<R::N, FOLD>(ss[0]);
       const float inv = rsqrtf(total + 1e-6f);
 #pragma unroll
       for (int j = 0; j < CJ; ++j)
@@ -794,10 +798,10 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
 #pragma unroll
           for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(m[s][j][e], m[cg][j][e], acc, 0, 0, 0);
         if constexpr (R::N == 16) {
-          gram[s][cg] = reduce_rows(acc);
+          gram[s][cg] = reduce_rows<FOLD>(acc);
         } else {
           float lo, hi;
-          reduce_rows8(acc, lo, hi);
+          reduce_rows8<FOLD>(acc, lo, hi);
           gram[s][cg] = (bq & 1) != 0 ? hi : lo;
         }
       }
@@ -953,11 +957,11 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
 #pragma unroll
       for (int cg = 0; cg < CG; ++cg) {
         if constexpr (R::N == 16) {
-          const float r = reduce_rows(acc[cg]);
+          const float r = reduce_rows<FOLD>(acc[cg]);
           y[cg] = g == 0 || bq == g ? r : y[cg];
         } else {
           float lo, hi;
-          reduce_rows8(acc[cg], lo, hi);
+          reduce_rows8<FOLD>(acc[cg], lo, hi);
           y[cg] = g == 0 || bq == 2 * g ? lo : y[cg];
           y[cg] = bq == 2 * g + 1 ? hi : y[cg];
         }
@@ -1076,11 +1080,14 @@ __device__ __forceinline__ void verify_wave(const VerifyArgs &a,
 // 256, 32 heads of V = 128, us with three waves / two: FP32 pages Q = 4, 128 rows
 // 152 / 103, Q = 1 99 / 90; BF16 pages Q = 8, 128 rows 100 / 94). So it is where FP32
 // activations meet the 16x16x1 form's accumulators on rows of 128 16-bit elements.
-// Shorter tiles at Q > 4 ask for two waves, which leaves a wave 256 registers and
-// none of the accumulation file: with one, every product was copied out of it
-// (FP32 K = 64, V = 192, Q = 8, 256 rows 122 / 113 us; K = V = 128, deferred, 64 rows
-// 71 / 68); the deferred FP16 kernels of K > 128 do not fit. At Q <= 4 the choice
-// made no difference but at K = 256, where one is faster (1 row 6.2 / 6.7).
+// Shorter tiles ask for two waves, which leaves a wave 256 registers and none of
+// the accumulation file: with one, products were copied out of it (Q = 8: FP32 K =
+// 64, V = 192, 256 rows 122 / 113 us; K = V = 128, deferred, 64 rows 71 / 68; Q = 4:
+// FP32 K = 256, 8 rows 12.7 / 12.0; FP16 K = 96, V = 192, 29 rows of 12 heads 11.0 /
+// 10.4). Not those it made slower, the ordinary BF16 tile of K = 128 at Q = 4 (32 rows
+// 14.6 / 15.1), nor 16 rows at Q <= 4 (no difference) and K > 128 at Q <= 2, where the
+// compiler spilled more scalars for it, nor the deferred FP16 kernels of K > 128 at
+// Q > 4, which do not fit.
 template <typename S, typename A, int KP>
 constexpr int verify_min_waves(int qm, int tile, bool defer) {
   using R = RowLanes<S, KP>;
@@ -1088,7 +1095,9 @@ constexpr int verify_min_waves(int qm, int tile, bool defer) {
   const int operands = (2 * qm + 3) / 4 * R::J * R::E;
   const bool wide_f32 = verify_wide<S, KP>(qm, defer, tile) && KP == 128 && sizeof(A) == 4;
   if (tile == 128) return buffers + operands <= 96 && !wide_f32 ? 3 : 2;
-  return qm == 8 && !(defer && KP == 256 && std::is_same_v<S, f16>) ? 2 : 1;
+  if (qm == 8) return defer && KP == 256 && std::is_same_v<S, f16> ? 1 : 2;
+  if (tile == 16 || (KP == 256 && qm <= 2)) return 1;
+  return !defer && KP == 128 && qm == 4 && std::is_same_v<S, bf16> ? 1 : 2;
 }
 template <typename S, typename A, int KP, int QM, bool DEFER, int TILE>
 __global__ __launch_bounds__(kVerifyThreads, (verify_min_waves<S, A, KP>(QM, TILE, DEFER))) void verify_kernel(
