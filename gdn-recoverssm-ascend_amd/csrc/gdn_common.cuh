@@ -212,18 +212,6 @@ __device__ __forceinline__ void store_b128_settled(gdn_u32x4 v, __amdgpu_buffer_
   asm volatile("s_nop %1" ::"v"(v), "n"(GDN_STORE_DATA_WAIT) : "memory");
 }
 
-// ----------------------------------------------------------------------------
-// Cross-lane sums inside aligned groups of 8 lanes with DPP (no LDS traffic):
-// quad_perm [1,0,3,2], quad_perm [2,3,0,1], then row_half_mirror, which pairs
-// lane i with lane 7-i of the same 8-lane half-row.
-// ----------------------------------------------------------------------------
-__device__ __forceinline__ float dpp_sum8(float x) {
-  x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false));
-  x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, false));
-  x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x141, 0xF, 0xF, false));
-  return x;
-}
-
 // Thread-local error message set by the host entry points.
 void set_error(const char *fmt, ...);
 
