@@ -17,10 +17,10 @@ static bool float_dt_ok(int32_t dt) { return dt == GDN_DT_F32 || dt == GDN_DT_BF
 // and 192 were measured too).
 //
 // Ordinary verify, tiles of 16 / 64 / 128 rows:
-//   * 16 rows up to 1536 waves (Q > 4: 1280), one and a half a SIMD. Q = 4: 4 rows
-//     6.0 / 7.4 / 10.7, 8 rows 9.4 / 7.8 / 11.0; BF16 4 rows 5.4 / 7.4 / 10.7, 8 rows 7.7
-//     / 7.7 / 10.8; K = 64, V = 192, 4 rows (1536) 5.8 / 6.8 / 8.7; Q = 8: 4 rows 8.6 / 11.6
-//     / 17.1, 8 rows 13.0 / 12.0 / 17.4.
+//   * 16 rows up to 1280 waves, a quarter more than SIMDs, rows of K <= 64 at Q <= 4 up
+//     to 1536. Q = 4: 4 rows 6.0 / 7.4 / 10.7, 6 rows (1536) 8.1 / 7.8, 8 rows 9.4 / 7.8 /
+//     11.0; BF16 4 rows 5.4 / 7.4 / 10.7, 8 rows 7.7 / 7.7 / 10.8; K = 64, V = 192, 4 rows
+//     (1536) 5.8 / 6.8 / 8.7; Q = 8: 4 rows 8.6 / 11.6 / 17.1, 8 rows 13.0 / 12.0 / 17.4.
 //   * V <= 32: a longer tile is mostly padding (256 rows 41 / 43 / 58).
 //   * FP32 pages of K > 64 at Q = 1, where a wave's own reads are a fraction of its
 //     tile: 16 rows up to 12288 waves (24 rows 13.5 / 15.4 / 16.0, 48 rows 23.1 / 25.5 /
@@ -56,7 +56,7 @@ static int verify_tile(int64_t rows, int64_t value_heads, int64_t K, int64_t V, 
     return !f32 || qm == 8 || waves(64) <= 3072 ? 64 : 32;
   }
   const int64_t w16 = waves(16);
-  if (w16 <= (qm == 8 ? 1280 : 1536) || V <= 32) return 16;
+  if (w16 <= (qm < 8 && K <= 64 ? 1536 : 1280) || V <= 32) return 16;
   if (f32 && K > 64 && qm == 1 && w16 <= (K > 128 ? 4096 : 12288)) return 16;
   if (f32 && K > 64 && K <= 128 && qm == 2 && w16 >= 4096 && w16 <= 8192) return 16;
   if ((V - 1) % 128 < 64) return 64;

@@ -38,7 +38,7 @@ def _tile(B, HV, K, V, Q, state=torch.float32):
 
 
 LINES = [  # (value heads, K, V, Q, largest batch on one side, its tile, the next batch's)
-    (32, 128, 128, 4, 6, 16, 64), (32, 128, 120, 4, 40, 64, 128), (32, 128, 120, 8, 5, 16, 64), (32, 128, 120, 8, 16, 64, 128),
+    (32, 128, 128, 4, 5, 16, 64), (32, 128, 120, 4, 40, 64, 128), (32, 128, 120, 8, 5, 16, 64), (32, 128, 120, 8, 16, 64, 128),
     (32, 128, 128, 1, 48, 16, 128), (32, 256, 120, 1, 16, 16, 64), (32, 128, 120, 1, 48, 16, 128),
     (32, 64, 120, 1, 6, 16, 64), (32, 128, 120, 2, 15, 64, 16), (32, 128, 120, 2, 32, 16, 64),
 ]

@@ -12,7 +12,7 @@ def verify_tile(rows, value_heads, K, V, f32, qm, deferred):
         if waves(32) <= 3072 or (V - 1) % 64 < 32:
             return 32
         return 64 if not f32 or qm == 8 or waves(64) <= 3072 else 32
-    if waves(16) <= (1280 if qm == 8 else 1536) or V <= 32:
+    if waves(16) <= (1536 if qm < 8 and K <= 64 else 1280) or V <= 32:
         return 16
     if f32 and K > 64 and qm == 1 and waves(16) <= (4096 if K > 128 else 12288):
         return 16
