@@ -45,15 +45,19 @@ static bool float_dt_ok(int32_t dt) { return dt == GDN_DT_F32 || dt == GDN_DT_BF
 //     V = 96, 128 rows 33.3 / 34.4 / 38.9).
 //   * 64 rows for 16-bit pages and Q > 4, bound by instructions that repeat per tile
 //     (BF16 Q = 4, 256 rows 171 / 124 / 114; Q = 8, 64 rows 92 / 78 / 68, 256 rows 335 / 273 /
-//     233); else while its waves stay within 3072 (32 rows 34.3 / 31.5 / 30.0), and 32
-//     rows past that (64 rows 60.8 / 57.6 / 60.0, 128 rows 112 / 104 / 104; 48 layers of 128
-//     rows took 5083 us at 32 rows and 5185 at 64; 256 rows 210 / 198 / 193 to 199).
+//     233); else while its waves stay within 3072 (32 rows 34.3 / 31.5 / 30.0), 32 rows
+//     past that (64 rows 60.8 / 57.6 / 60.0, 128 rows 112 / 104 / 104; 48 layers of 128 rows
+//     took 5076 us at 32 rows and 5150 at 64), and at Q = 4 with 64 < K <= 128 64 rows
+//     again past 16384 waves of 32 (192 rows 151 / 149; 256 rows 198 / 193 to 199, and as
+//     single steps after five warm-up ones 214 to 221 / 202 to 204; Q = 1, 256 rows 143 / 150;
+//     K = 256, 256 rows 32-row tiles 4% ahead).
 static int verify_tile(int64_t rows, int64_t value_heads, int64_t K, int64_t V, bool f32, int qm, bool deferred) {
   auto waves = [&](int tile) { return rows * value_heads * ((V + tile - 1) / tile); };
   if (deferred) {
     if (waves(16) <= (qm == 8 ? 1280 : 3072) || V <= 16) return 16;
     if (waves(32) <= 3072 || (V - 1) % 64 < 32) return 32;
-    return !f32 || qm == 8 || waves(64) <= 3072 ? 64 : 32;
+    if (!f32 || qm == 8 || waves(64) <= 3072) return 64;
+    return qm == 4 && K > 64 && K <= 128 && waves(32) > 16384 ? 64 : 32;
   }
   const int64_t w16 = waves(16);
   if (w16 <= (qm < 8 && K <= 64 ? 1536 : 1280) || V <= 32) return 16;

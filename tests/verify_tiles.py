@@ -11,7 +11,9 @@ def verify_tile(rows, value_heads, K, V, f32, qm, deferred):
             return 16
         if waves(32) <= 3072 or (V - 1) % 64 < 32:
             return 32
-        return 64 if not f32 or qm == 8 or waves(64) <= 3072 else 32
+        if not f32 or qm == 8 or waves(64) <= 3072:
+            return 64
+        return 64 if qm == 4 and 64 < K <= 128 and waves(32) > 16384 else 32
     if waves(16) <= (1536 if qm < 8 and K <= 64 else 1280) or V <= 32:
         return 16
     if f32 and K > 64 and qm == 1 and waves(16) <= (4096 if K > 128 else 12288):
